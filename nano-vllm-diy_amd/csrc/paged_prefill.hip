@@ -8,37 +8,33 @@
 // from fresh rows at cu_seqlens_k (flat, all-fresh prompts).
 //
 // Work unit: 256 query rows = TM = 256 / G query tokens x the G query heads of one kv
-// head g, so each K/V tile staged in LDS serves the whole GQA group. A work-group of eight
-// wavefronts (two per SIMD, one work-group per CU) owns the unit; wavefront w owns rows
-// 32 w .. 32 w + 31, which are 32 consecutive tokens of one head (TM >= 32 for every GQA
-// group built). All eight wavefronts pass one barrier per K/V tile, so the two wavefronts
-// of a SIMD run the loop in step; what overlaps one's softmax with the other's MFMAs is
-// only the hardware's interleaving of their instructions.
+// head g, so each K/V tile staged in LDS serves the whole GQA group. A work-group of four
+// wavefronts (one per SIMD, one work-group per CU, the whole register file) owns the unit; a
+// wavefront owns two blocks of 32 rows, each 32 consecutive tokens of one head (TM >= 32 for
+// every GQA group built).
 //
 // Three launches, all sized on the host without reading device memory:
 //   1. plan (one work-group): reads cu_seqlens_q/k, counts each unit's key tiles under
 //      its causal limit, picks a split size T = max(8, kSplitNum / kSplitDen x total tiles
 //      / pool) tiles and writes the work list: every unit longer than T is cut into equal
 //      key ranges. Long items come first (four length buckets, longest first).
-//   2. prefill (a persistent pool of one work-group per CU): each work-group claims items
-//      from the sub-queue of its XCD (item i belongs to sub-queue i mod 8, which for 8 kv
-//      heads is kv head i mod 8, so a head's K/V stays in one XCD's L2), then steals from
-//      the other sub-queues. An unsplit item writes bf16 rows; a split item writes its
-//      fp32 numerators and (max, sum) per row.
+//   2. prefill (a persistent pool of one work-group per CU): each work-group starts on the item
+//      of its own index, then claims items from the sub-queue of its XCD (item i belongs to
+//      sub-queue i mod 8, which for 8 kv heads is kv head i mod 8, so a head's K/V stays in one
+//      XCD's L2), then steals from the other sub-queues. An unsplit item writes bf16 rows; a
+//      split item writes its own output in bf16 and (max, sum) per row.
 //   3. merge: combines the partials of every split unit, then the decode rows' partials
 //      left by the call's decode launch (paged_decode.hip), which needs no combine launch.
 // The split bounds the longest chain of dependent tiles (a long cached prefix would
 // otherwise keep one work-group busy long after the rest of the GPU has finished).
 //
-// Per 64-key tile, per wavefront and 32-row block:
-//   S^T (64 keys x 32 rows) = K (64 x 128) . Q^T (128 x 32)    16 v_mfma_f32_32x32x16_bf16
-//   online softmax down each column (a lane owns one query row; the two lane halves
-//   exchange through v_permlane32_swap)
-//   O^T (128 x 32)         += V^T (128 x 64) . P^T (64 x 32)   16 v_mfma_f32_32x32x16_bf16
-// K and V tiles move global -> registers -> LDS: two LDS stages of 16 KiB per operand
-// (sK[2], sV[2]); at step n the loads of tile n + 2 are issued, tile n is computed and
-// tile n + 1 is written from registers into the other stage. The P.V A operand comes
-// from the LDS transpose read. P^T never leaves registers: the
+// Per step of 32 keys (half a tile), per wavefront and 32-row block:
+//   S^T (32 keys x 32 rows) = K (32 x 128) . Q^T (128 x 32)    8 v_mfma_f32_32x32x16_bf16
+//   P = 2^(S - reference of the row) (a lane owns one query row)
+//   O^T (128 x 32)         += V^T (128 x 32) . P^T (32 x 32)   8 v_mfma_f32_32x32x16_bf16
+// The three parts of consecutive steps run as one instruction stream (pf_iteration). K and V
+// tiles go from memory to LDS without registers (global_load_lds), K four tiles and V three tiles
+// deep. The P.V A operand comes from the LDS transpose read. P^T never leaves registers: the
 // S^T accumulator layout already holds, per lane, the keys the P.V B operand needs once
 // the k-order of the instruction is permuted (same permutation on the V side).
 #include <algorithm>
@@ -78,11 +74,12 @@ constexpr int kMergeBatch = 8;         // merge: splits whose (max, sum) load in
 #endif
 constexpr int kMergeLoads = PK_MERGE_LOADS;  // merge: splits whose outputs load in one batch
 #ifndef PK_PREFILL_BUCKETS
-#define PK_PREFILL_BUCKETS 4
+#define PK_PREFILL_BUCKETS 8
 #endif
-constexpr int kBuckets = PK_PREFILL_BUCKETS;  // length buckets of the work list (longest first)
+// length buckets of the work list (longest first): 4 -> 8 took the dense prompts 144.4 -> 141.6 us
+// and the long chunks 605 -> 594 us; 16 gave 146.3 and 594
+constexpr int kBuckets = PK_PREFILL_BUCKETS;
 constexpr float kLazyLog2 = 8.f;       // reference max moves only when exceeded by 2^8
-constexpr int kStages = 2;             // K and V LDS stages of the prefill kernel
 
 typedef short v4i16 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) char lds_char;
@@ -170,27 +167,6 @@ __device__ __forceinline__ void load_rows(const uint16_t* kbase, const uint16_t*
     R.k[i] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(kbase) + l.k[i]);
     R.v[i] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(vbase) + l.v[i]);
   }
-}
-
-template <bool PAGED>
-__device__ __forceinline__ void load_tile_regs(const AttnArgs& a, int b, int k0, int Lk, int g, int bt_lane, int wave,
-                                               int lane, int t0, const LoadLanes& full_lanes, KvRegs& R) {
-  const uint16_t* kbase;
-  const uint16_t* vbase;
-  if constexpr (PAGED) {
-    const int j = t0 / a.block_size;  // block_size % 64 == 0: the tile sits inside one block
-    const int blk = j < kWave ? __builtin_amdgcn_readlane(bt_lane, j)
-                              : __builtin_amdgcn_readfirstlane(a.block_table[(int64_t)b * a.bt_stride + j]);
-    const int off = t0 % a.block_size;
-    kbase = a.k + (int64_t)blk * a.k_block_stride + (int64_t)off * a.k_row_stride;
-    vbase = a.v + (int64_t)blk * a.v_block_stride + (int64_t)off * a.v_row_stride;
-  } else {
-    kbase = a.k + (int64_t)(k0 + t0) * a.k_row_stride;
-    vbase = a.v + (int64_t)(k0 + t0) * a.v_row_stride;
-  }
-  kbase += g * kHeadDim;
-  vbase += g * kHeadDim;
-  load_rows(kbase, vbase, (t0 + kTileKeys <= Lk) ? full_lanes : load_lanes(a, wave, lane, Lk - 1 - t0), R);
 }
 
 __device__ __forceinline__ void store_tile_lds(const KvRegs& R, lds_char* kdst, lds_char* vdst, int wave, int lane) {
@@ -446,25 +422,37 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const AttnAr
   constexpr int W = kPlanThreads / kWave;
   __shared__ long long red[W];
   __shared__ int cur[kBuckets + 2];  // bucket cursors, partial-group cursor, merge cursor
-  // (Lq, Lk) of up to kPlanCache sequences, so passes 2 and 3 skip the global round trip
-  __shared__ int2 dims[kPlanCache];
+  // (sequence, Lq, Lk) of the prefill sequences among the first kPlanCache, in any order: the
+  // passes read them from LDS and do not walk the decode rows of a mixed batch (128 of them beside
+  // 8 chunks: nine rounds of the wavefronts per pass instead of one, 9.5 us for the plan)
+  __shared__ int4 dims[kPlanCache];
+  __shared__ int listed;
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave = tid / kWave;
   const int S = a.num_seqs;
   const int hkv = a.num_kv_heads;
 
+  if (tid == 0) listed = 0;
+  __syncthreads();
   for (int b = tid; b < min(S, kPlanCache); b += kPlanThreads) {
     const SeqDims d = seq_dims<TM>(a, b);
-    dims[b] = make_int2(d.Lq, d.Lk);
+    if (d.nq > 0) dims[atomicAdd(&listed, 1)] = make_int4(b, d.Lq, d.Lk, 0);
   }
   __syncthreads();
-  auto dims_of = [&](int b) {
-    if (b >= kPlanCache) return seq_dims<TM>(a, b);
+  const int nlist = listed;
+  const int nseq = nlist + max(0, S - kPlanCache);  // entries of the passes: the list, then the rest
+  auto dims_of = [&](int i, int& b) {
+    if (i >= nlist) {
+      b = kPlanCache + i - nlist;
+      return seq_dims<TM>(a, b);
+    }
     SeqDims d;
     d.q0 = d.k0 = 0;  // not used by the plan
-    d.Lq = dims[b].x;
-    d.Lk = dims[b].y;
+    const int4 e = dims[i];
+    b = e.x;
+    d.Lq = e.y;
+    d.Lk = e.z;
     d.P = d.Lk - d.Lq;
     d.nq = (d.Lq <= 1 || d.Lk <= 0) ? 0 : min((d.Lq + TM - 1) / TM, a.prefill_qtiles);
     return d;
@@ -472,8 +460,9 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const AttnAr
 
   // pass 1: total key tiles over all units
   long long tiles = 0;
-  for (int b = wave; b < S; b += W) {
-    const SeqDims d = dims_of(b);
+  for (int i = wave; i < nseq; i += W) {
+    int b;
+    const SeqDims d = dims_of(i, b);
     for (int qt = lane; qt < d.nq; qt += kWave) tiles += unit_tiles<TM, CAUSAL>(d, qt);
   }
 #pragma unroll
@@ -492,8 +481,9 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const AttnAr
                              (kSplitNum * (work / kSplitDen) + a.pf_slots - 1) / a.pf_slots + 1));
 
   // pass 2: groups per length bucket
-  for (int b = wave; b < S; b += W) {
-    const SeqDims d = dims_of(b);
+  for (int i = wave; i < nseq; i += W) {
+    int b;
+    const SeqDims d = dims_of(i, b);
     for (int qt = lane; qt < d.nq; qt += kWave) {
       const int t = unit_tiles<TM, CAUSAL>(d, qt);
       const int n = unit_splits(t, T);
@@ -514,8 +504,9 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const AttnAr
 
   // pass 3: emit one entry per group; kv heads are expanded by index (item i = head i % hkv
   // of group i / hkv)
-  for (int b = wave; b < S; b += W) {
-    const SeqDims d = dims_of(b);
+  for (int i = wave; i < nseq; i += W) {
+    int b;
+    const SeqDims d = dims_of(i, b);
     for (int qt = lane; qt < d.nq; qt += kWave) {
       const int t = unit_tiles<TM, CAUSAL>(d, qt);
       const int n = unit_splits(t, T);
@@ -537,7 +528,8 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const AttnAr
   // LDS-only: the counts in cur are final; the work-list stores need not complete before the
   // queue header's (the prefill kernel, a later launch, reads both)
   lds_barrier();
-  if (tid < 8) a.pf_queue[tid * kPrefillQueueStride] = 0;
+  // sub-queue x starts behind the items that its work-groups take without a claim
+  if (tid < 8) a.pf_queue[tid * kPrefillQueueStride] = (a.pf_slots - tid + 7) / 8;
   if (tid == 0) {
     a.pf_queue[kPrefillQueueMeta] = (int)(min((int64_t)tot, (int64_t)a.pf_item_cap) * hkv);
     a.pf_queue[kPrefillQueueMeta + 1] = (int)(min((int64_t)cur[kBuckets + 1], (int64_t)a.pf_merge_cap) * hkv);
@@ -545,198 +537,462 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const AttnAr
   }
 }
 
-// One work item: kv head g of group `it` = (sequence b, query tile qt, key tiles [tb, te),
-// partial group or -1). The caller's hooks run at three points, which the kernel uses to
-// claim and prefetch the next item: last_step when the last key tile starts, after_tiles
-// after the last tile's barrier (before the epilogue), after_epilogue after its stores.
-template <int G, bool PAGED, bool CAUSAL, class LastStep, class AfterTiles, class AfterEpilogue>
-__device__ __forceinline__ void prefill_item(const AttnArgs& a, const int4 it, const int g, const int cuv,
-                                             const int bt_lane, lds_char* const (&KS)[kStages],
-                                             lds_char* const (&VS)[kStages],
-                                             int wave, int lane,
-                                             LastStep&& last_step, AfterTiles&& after_tiles,
-                                             AfterEpilogue&& after_epilogue) {
+// ---- The prefill kernel's tile loop --------------------------------------------------------
+// What bounded the loop before (eight wavefronts of one row block, phases QK - softmax - PV with
+// a barrier per tile, 4600 cycles per 64-key tile for 2048 cycles of MFMA): the two wavefronts of
+// a SIMD passed the phases together, so the MFMA, vector and LDS work added up, and every
+// wavefront read the whole tile from LDS (256 KiB per tile and CU at 128 B per cycle: as long as
+// the MFMAs). Two row blocks per wavefront halve the LDS reads, and one wavefront per SIMD has
+// the registers (O 128, Q 64, two steps' scores 64 and P 32) to run three steps' parts beside
+// each other. What the loop then needs, measured per instruction (cycles, one wavefront): an MFMA
+// takes 32, up to five independent vector instructions beside it are free, a sixth and further
+// ones cost 4-5, a vector instruction that uses the previous one's result 8, an exponential 8,
+// v_dot2 (which the MFMA pipe executes too) 17, an LDS read beside a full slot 4. Hence: no
+// instruction uses a result of its own slot; sums are additions, not v_dot2; no running max (one
+// reference per row and item with 2^124 of room, checked by the sum at the end); K and V bypass
+// the registers. Steady tile 4600 -> 3000 cycles; 16 chunks of 1024 over 4096-token prefixes
+// (618 GFLOP) 647-670 -> 584-617 us per call with the 24 us store (kernel alone 692 -> 591 us in a
+// trace), at a clock that now falls with the load: an 8192^3 matrix product of the vendor's
+// library reaches 1.21 PFLOP/s here. A mixed step of 128 decodes and 8 chunks of 512 302.7 ->
+// 300.3 us, 31 dense prompts of 16384 tokens 150.9 -> 149.8 us: short items are bound by their
+// start and end (about 20000 of an average item's 45000 cycles).
+constexpr int kPfWaves = 4;                      // one wavefront per SIMD, 64 query rows each
+constexpr int kPfThreads = kPfWaves * kWave;
+constexpr int kPfRB = kPrefillRows / (32 * kPfWaves);  // 32-row blocks per wavefront
+// LDS: four K and three V stages; the stages that an item's first loads do not use (K 3, V 1, V 2)
+// and one tile more hold its Q rows on their way to registers, and a last tile the output rows on
+// their way out.
+constexpr int kLdsK0 = 0, kLdsK1 = kTileBytes, kLdsK2 = 2 * kTileBytes, kLdsK3 = 4 * kTileBytes;
+constexpr int kLdsV0 = 3 * kTileBytes, kLdsV1 = 5 * kTileBytes, kLdsV2 = 6 * kTileBytes;
+constexpr int kLdsQ = 4 * kTileBytes, kLdsO = 8 * kTileBytes;
+constexpr int kPfLdsBytes = 9 * kTileBytes;
+constexpr int kPfAhead = 3;                      // operands read this many ahead of their MFMAs
+constexpr int kStepKeys = 32;                    // keys per pipeline step (half a tile)
+constexpr int kPfLoads = kTileKeys / kPfWaves / 4;     // 16-byte loads per lane, operand and tile
+constexpr float kHeadroomLog2 = 60.f;            // first step's largest p is 2^-60 ...
+constexpr float kSumLimit = 18446744073709551616.f;  // ... and a row's sum may grow to 2^64
+
+static_assert(kPfLoads == 4, "stage_tile issues four loads per operand");
+
+// Byte offsets of the tile rows this lane moves (row r clamped to `last`), for stage_tile.
+template <bool V>
+__device__ __forceinline__ void stage_offsets(int row_stride, int wave, int lane, int last, int (&off)[kPfLoads]) {
+  const int slot = lane & 15;
+#pragma unroll
+  for (int i = 0; i < kPfLoads; ++i) {
+    const int r = 4 * kPfLoads * wave + 4 * i + (lane >> 4);
+    const int c = V ? v_chunk(r, slot) : slot ^ (r & 15);
+    off[i] = (min(r, last) * row_stride + c * 8) * 2 + 1024 * (kPfLoads - 1 - i);
+  }
+}
+
+// The wavefront's rows of a tile, memory to LDS without registers: lane l of load i moves 16
+// bytes from base + off[i] - 1024 (3 - i) to lds + 1024 i + 16 l. (The instruction's offset
+// moves both addresses; off carries the correction.)
+__device__ __forceinline__ void stage_tile(const char* base, const int (&off)[kPfLoads], int lds) {
+  const uint64_t u = (uint64_t)(base - 1024 * (kPfLoads - 1));
+  const uint64_t b = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)u) |
+                     (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(u >> 32)) << 32;
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, %5\n\t"
+      "global_load_lds_dwordx4 %2, %5 offset:1024\n\t"
+      "global_load_lds_dwordx4 %3, %5 offset:2048\n\t"
+      "global_load_lds_dwordx4 %4, %5 offset:3072"
+      :
+      : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "s"(b)
+      : "m0", "memory");
+}
+
+// One of stage_tile's loads.
+template <int I>
+__device__ __forceinline__ void stage_load(const char* base, int off, int lds) {
+  const uint64_t u = (uint64_t)(base - 1024 * (kPfLoads - 1));
+  const uint64_t b = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)u) |
+                     (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(u >> 32)) << 32;
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, %2 offset:%c3"
+      :
+      : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(off), "s"(b), "i"(1024 * I)
+      : "m0", "memory");
+}
+
+// 16 bytes per lane from per-lane addresses to lds + 16 l.
+__device__ __forceinline__ void load_lds16(const uint16_t* src, int lds) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, off"
+      :
+      : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(src)
+      : "m0", "memory");
+}
+
+// Waits until at most N of this wavefront's vector memory operations are in flight.
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
+}
+
+// The wavefront's state over an item. O and the second row block's Q live in accumulation
+// registers, everything else in architectural ones.
+struct PfState {
+  bf16x8 q[kPfRB][kHeadDim / 16];
+  f32x16 o[kPfRB][4];
+  f32x16 s[2][kPfRB];          // scores of steps of either parity
+  u32x4 p[2][kPfRB][2];        // P (bf16 pairs) of steps of either parity
+  bf16x8 kf[kPfAhead];         // K operands read ahead
+  float nm[kPfRB];             // minus the reference max of the exponentials
+  float l[kPfRB];              // row sums over this lane's keys
+};
+
+__device__ __forceinline__ bf16x8 read_k(const lds_char* sK, const TileLanes& tl, int kb) {
+  return *reinterpret_cast<const __attribute__((address_space(3))) bf16x8*>(sK + tl.k(kb));
+}
+__device__ __forceinline__ bf16x8 read_v(const lds_char* sV, const TileLanes& tl, int f) {
+  const lds_char* p = sV + tl.v(f & 3) + (f >> 2) * 16 * kRowBytes;
+  const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      const_cast<lds_v4i16*>(reinterpret_cast<const lds_v4i16*>(p)));
+  const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      const_cast<lds_v4i16*>(reinterpret_cast<const lds_v4i16*>(p + 8 * kRowBytes)));
+  return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+// The MFMAs are written out because the compiler keeps one register kind per kernel for their
+// results: S, which the vector instructions read, belongs in architectural registers and O, which
+// nothing reads before the item's end, in accumulation registers. The compiler does not add the
+// wait states of an MFMA that it does not know, so the order of the stream provides them: a score
+// is read 16 MFMAs after the last that wrote it, P is used 16 MFMAs after its conversion, K, Q
+// and V operands come from LDS reads (which are waited for); pf_iteration's scheduling barriers
+// keep that order.
+// S += K Q^T with S in architectural registers, Q in architectural (row block 0) or accumulation
+// registers (row block 1).
+__device__ __forceinline__ void mfma_s(f32x16& s, const bf16x8& k, const bf16x8& q, bool first, int rb) {
+  if (first && rb == 0)
+    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(s) : "v"(k), "v"(q));
+  else if (first)
+    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(s) : "v"(k), "a"(q));
+  else if (rb == 0)
+    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(s) : "v"(k), "v"(q));
+  else
+    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(s) : "v"(k), "a"(q));
+}
+
+// O += V^T P^T with O in accumulation registers.
+__device__ __forceinline__ void mfma_o(f32x16& o, const bf16x8& v, const u32x4& p) {
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(o) : "v"(v), "v"(p));
+}
+
+// The first softmax of an item (step 0): the reference is the row's max over the step's keys
+// raised by kHeadroomLog2, P = 2^(s - reference) in bf16. Later steps keep the reference.
+__device__ __forceinline__ void softmax_first(PfState& st, int t0, const int (&lim)[kPfRB], float scale_log2,
+                                              int half) {
+#pragma unroll
+  for (int rb = 0; rb < kPfRB; ++rb) {
+    float s[16];
+#pragma unroll
+    for (int rr = 0; rr < 16; ++rr)
+      s[rr] = t0 + 8 * (rr >> 2) + 4 * half + (rr & 3) > lim[rb] ? -INFINITY : st.s[0][rb][rr];
+    float t = s[0];
+#pragma unroll
+    for (int rr = 1; rr < 16; ++rr) t = fmaxf(t, s[rr]);
+    t = swap_halves_max(t) * scale_log2;
+    const float nm = t == -INFINITY ? 0.f : -t - kHeadroomLog2;
+    float ps = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; i += 2) {
+      const float p0 = exp2_fast(__builtin_fmaf(s[i], scale_log2, nm));
+      const float p1 = exp2_fast(__builtin_fmaf(s[i + 1], scale_log2, nm));
+      const bf16x2 pr = {static_cast<__bf16>(p0), static_cast<__bf16>(p1)};
+      st.p[0][rb][i >> 3][(i & 7) >> 1] = __builtin_bit_cast(uint32_t, pr);
+      ps += p0 + p1;
+    }
+    st.nm[rb] = nm;
+    st.l[rb] = ps;
+  }
+}
+
+// Pipeline iteration i of a wavefront: S(i + 1) = K Q^T of step i + 1, the softmax of step i and
+// O += V^T P^T of step i - 1, three independent streams; CUR = i & 1. 32 slots of one MFMA each
+// (16 QK, then 16 PV), and beside it the slot's share of the LDS reads (kPfAhead operands ahead;
+// the next iteration's first K operands at the end), of the softmax and, with STAGE, of the loads
+// of a tile (from `src`, offsets `soff`, to LDS `lds`). MASK: keys past a row's limit count 0.
+template <int CUR, bool MASK, bool STAGE>
+__device__ __forceinline__ void pf_iteration(PfState& st, const lds_char* sK, const lds_char* sKn, const lds_char* sV,
+                                             const TileLanes& tl, int t0, const int (&lim)[kPfRB],
+                                             float scale_log2, int half, const char* src,
+                                             const int (&soff)[kPfLoads], int lds) {
+  constexpr int NXT = CUR ^ 1;
+  constexpr int KB = kHeadDim / 16;
+  constexpr int NE = 16 * kPfRB;  // scores per lane
+  bf16x8 kf[KB], vf[8];
+  float ps[kPfRB];
+  float x[NE];  // a score on its way to p
+#pragma unroll
+  for (int rb = 0; rb < kPfRB; ++rb) {
+    ps[rb] = 0.f;
+  }
+#pragma unroll
+  for (int j = 0; j < kPfAhead; ++j) kf[j] = st.kf[j];
+  // elements started by the end of slot s: 32 of them in 29 slots, so the last is packed in slot 31
+  const auto nf = [](int s) { return s < 0 ? 0 : (s + 1) * NE >= 29 * NE ? NE : ((s + 1) * NE + 28) / 29; };
+#pragma unroll
+  for (int sl = 0; sl < 32; ++sl) {
+    // LDS reads
+    if (sl < 16 && (sl & 1) == 0 && sl / 2 + kPfAhead < KB)
+      kf[sl / 2 + kPfAhead] = read_k(sK, tl, sl / 2 + kPfAhead);
+    const int f = sl - (16 - 2 * kPfAhead);
+    if (f >= 0 && (f & 1) == 0 && f / 2 < 8) vf[f / 2] = read_v(sV, tl, f / 2);
+    const int j = sl - (29 - kPfAhead);
+    if (j >= 0 && j < kPfAhead) st.kf[j] = read_k(sKn, tl, j);
+    // the tile's loads, between the others
+    if constexpr (STAGE) {
+      if (sl == 3) stage_load<0>(src, soff[0], lds);
+      if (sl == 7) stage_load<1>(src, soff[1], lds);
+      if (sl == 11) stage_load<2>(src, soff[2], lds);
+      if (sl == 15) stage_load<3>(src, soff[3], lds);
+    }
+    // MFMAs
+    if (sl < 16) {
+      mfma_s(st.s[NXT][sl & 1], kf[sl / 2], st.q[sl & 1][sl / 2], sl < 2, sl & 1);
+    } else {
+      const int fv = (sl - 16) / 2, rb = sl & 1;
+      mfma_o(st.o[rb][fv & 3], vf[fv], st.p[NXT][rb][fv >> 2]);
+    }
+    // softmax: the scale and reference of some elements, the exponentials of those of the slot
+    // before, sum and packing of those of the slot before that
+#pragma unroll
+    for (int e = nf(sl - 4); e < nf(sl - 3); ++e) {
+      ps[e >> 4] += x[e];
+      asm volatile("" ::"v"(ps[e >> 4]));  // here, not after the loop
+      if (e & 1) {
+        const bf16x2 pr = {static_cast<__bf16>(x[e - 1]), static_cast<__bf16>(x[e])};
+        st.p[CUR][e >> 4][(e & 15) >> 3][(e & 7) >> 1] = __builtin_bit_cast(uint32_t, pr);
+      }
+    }
+#pragma unroll
+    for (int e = nf(sl - 1); e < nf(sl); ++e) {
+      const int rr = e & 15, rb = e >> 4;
+      float v = st.s[CUR][rb][rr];
+      if constexpr (MASK) v = t0 + 8 * (rr >> 2) + 4 * half + (rr & 3) > lim[rb] ? -INFINITY : v;
+      x[e] = __builtin_fmaf(v, scale_log2, st.nm[rb]);
+    }
+#pragma unroll
+    for (int e = nf(sl - 2); e < nf(sl - 1); ++e) {
+      x[e] = exp2_fast(x[e]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for (int rb = 0; rb < kPfRB; ++rb) {
+    st.l[rb] += ps[rb];
+    // S is final here (the MFMAs that wrote it are 16 MFMAs back), and P is computed before here
+    asm volatile("" : "+v"(st.s[NXT][rb]), "+v"(st.p[CUR][rb][0]), "+v"(st.p[CUR][rb][1]));
+  }
+}
+
+// Cursor over an item's key tiles: the tile's first K and V row of kv head g and its first key.
+template <bool PAGED>
+struct TileCursor {
+  const char *k, *v;
+  int t0, last, j, off;
+  int64_t kstep, vstep;
+  __device__ __forceinline__ void to_block(const AttnArgs& a, int b, int g, int bt_lane) {
+    const int blk = j < kWave ? __builtin_amdgcn_readlane(bt_lane, j)
+                              : __builtin_amdgcn_readfirstlane(a.block_table[(int64_t)b * a.bt_stride + j]);
+    k = reinterpret_cast<const char*>(a.k + (int64_t)blk * a.k_block_stride + (int64_t)off * a.k_row_stride +
+                                      g * kHeadDim);
+    v = reinterpret_cast<const char*>(a.v + (int64_t)blk * a.v_block_stride + (int64_t)off * a.v_row_stride +
+                                      g * kHeadDim);
+  }
+  __device__ __forceinline__ void init(const AttnArgs& a, int b, int g, int k0, int tbase, int ntiles, int bt_lane) {
+    t0 = tbase;
+    last = tbase + (ntiles - 1) * kTileKeys;
+    kstep = a.k_row_stride * (2 * kTileKeys);
+    vstep = a.v_row_stride * (2 * kTileKeys);
+    j = off = 0;
+    k = reinterpret_cast<const char*>(a.k + g * kHeadDim);
+    v = reinterpret_cast<const char*>(a.v + g * kHeadDim);
+    if constexpr (PAGED) {
+      j = tbase / a.block_size;  // block_size % 64 == 0: a tile sits inside one block
+      off = tbase - j * a.block_size;
+      if (ntiles > 0) to_block(a, b, g, bt_lane);
+    } else {
+      k += (int64_t)(k0 + tbase) * a.k_row_stride * 2;
+      v += (int64_t)(k0 + tbase) * a.v_row_stride * 2;
+    }
+  }
+  // To the next tile; the last one stays.
+  __device__ __forceinline__ void advance(const AttnArgs& a, int b, int g, int bt_lane) {
+    if (t0 < last) step(a, b, g, bt_lane);
+  }
+  __device__ __forceinline__ void step(const AttnArgs& a, int b, int g, int bt_lane) {
+    t0 += kTileKeys;
+    k += kstep;
+    v += vstep;
+    if constexpr (PAGED) {
+      off += kTileKeys;
+      if (off == a.block_size) {
+        off = 0;
+        ++j;
+        to_block(a, b, g, bt_lane);
+      }
+    }
+  }
+};
+
+// The first row of row block rb of wavefront `wave`. A wavefront's two blocks hold the same tokens
+// of two heads where the unit has two heads (G > 1), so that the causal limit crosses few of its
+// steps; G = 1: neighbouring tokens.
+template <int G>
+__device__ __forceinline__ int block_row(int wave, int rb) {
+  constexpr int NB = kPrefillRows / G / 32;  // blocks of a head
+  return 32 * (NB == 8 ? 2 * wave + rb : wave % NB + NB * rb + 2 * NB * (wave / NB));
+}
+
+
+// A work item: kv head g of group (sequence b, query tile qt, key tiles [tb, te), partial group),
+// with the sequence's bounds.
+struct PfItem {
+  int b, qt, tb, te, part, g, q0, Lq, k0, Lk;
+};
+
+// From the work-list entry and the sequence's bounds (cu_q[b], cu_q[b + 1], cu_k[b], cu_k[b + 1]).
+// The work list is trusted only as far as the buffers reach: an entry naming a sequence or key
+// tiles outside this call (a workspace overwritten by an overlapping call) becomes an item
+// without rows or tiles.
+__device__ __forceinline__ PfItem make_item(const AttnArgs& a, int idx, const int4& grp, const int4& cu) {
+  PfItem it;
+  it.g = __builtin_amdgcn_readfirstlane(idx % a.num_kv_heads);
+  it.b = grp.x;
+  it.qt = grp.y;
+  it.tb = grp.z & 0xffff;
+  it.te = grp.z >> 16;
+  it.part = grp.w < 0 ? -1 : grp.w * a.num_kv_heads + it.g;
+  it.q0 = cu.x;
+  it.Lq = cu.y - cu.x;
+  it.k0 = cu.z;
+  it.Lk = min(cu.w - cu.z, a.max_seqlen_k);
+  if (it.b < 0 || it.b >= a.num_seqs || it.Lq <= 0 || it.tb > it.te ||
+      it.te > (it.Lk + kTileKeys - 1) / kTileKeys) {
+    it.b = it.qt = it.tb = it.te = it.q0 = it.Lq = it.k0 = it.Lk = 0;
+    it.part = -1;
+  }
+  return it;
+}
+
+// v, as a value of its own at every use: what is computed from it is computed again for every item
+// instead of being kept in registers through the tile loops.
+__device__ __forceinline__ int per_item(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
+// An item's tiles one after the other with a running row max (numerator and sum rescaled when it
+// moves by more than 2^kLazyLog2): what an item takes whose scores leave the range that one
+// reference covers. Ends with a barrier.
+template <int G, bool PAGED>
+__device__ __forceinline__ void prefill_item_safe(const AttnArgs& a, PfState& st, const PfItem& it, int bt_lane,
+                                                  const int (&lim)[kPfRB], lds_char* const smem, int wave, int lane) {
+  constexpr int TM = kPrefillRows / G;
+  const int b = it.b, g = it.g, k0 = it.k0, Lk = it.Lk, tbase = it.tb * kTileKeys, ntiles = it.te - it.tb;
+  const int half = lane >> 5;
+  // Q again (the tile loops' operands need not outlive them)
+#pragma unroll
+  for (int rb = 0; rb < kPfRB; ++rb) {
+    const int row = block_row<G>(wave, rb) + (lane & 31);
+    const int tok = min(it.qt * TM + row % TM, it.Lq - 1);
+    const uint16_t* qp = a.q + (int64_t)(it.q0 + tok) * a.q_row_stride + (g * G + row / TM) * kHeadDim + 8 * half;
+#pragma unroll
+    for (int kb = 0; kb < kHeadDim / 16; ++kb)
+      st.q[rb][kb] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(qp + kb * 16));
+  }
+  const TileLanes tl = tile_lanes(lane);
+  const int lds0 = (int)(uintptr_t)smem + 4 * kPfLoads * wave * kRowBytes;
+  TileCursor<PAGED> cur;
+  cur.init(a, b, g, k0, tbase, ntiles, bt_lane);
+  float m[kPfRB];
+  const float zero = __int_as_float(per_item(0));
+#pragma unroll
+  for (int rb = 0; rb < kPfRB; ++rb) {
+    m[rb] = -INFINITY;
+    st.l[rb] = 0.f;
+#pragma unroll
+    for (int md = 0; md < 4; ++md)
+#pragma unroll
+      for (int rr = 0; rr < 16; ++rr) st.o[rb][md][rr] = zero;
+  }
+#pragma unroll 1
+  for (int n = 0; n < ntiles; ++n) {
+    const int t0 = cur.t0;
+    int off[kPfLoads];
+    stage_offsets<false>((int)a.k_row_stride, wave, lane, min(kTileKeys, Lk - 1 - t0), off);
+    stage_tile(cur.k, off, lds0);
+    stage_offsets<true>((int)a.v_row_stride, wave, lane, min(kTileKeys, Lk - 1 - t0), off);
+    stage_tile(cur.v, off, lds0 + kTileBytes);
+    cur.advance(a, b, g, bt_lane);
+    wait_vm<0>();
+    lds_barrier();
+#pragma unroll 1
+    for (int hs = 0; hs < 2; ++hs) {
+      const lds_char* const sK = smem + hs * 32 * kRowBytes;
+      const lds_char* const sV = smem + kTileBytes + hs * 32 * kRowBytes;
+#pragma unroll
+      for (int rb = 0; rb < kPfRB; ++rb) {
+        f32x16 s[1];
+#pragma unroll
+        for (int rr = 0; rr < 16; ++rr) s[0][rr] = 0.f;
+#pragma unroll
+        for (int kb = 0; kb < kHeadDim / 16; ++kb)
+          s[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(read_k(sK, tl, kb), st.q[rb][kb], s[0], 0, 0, 0);
+        bf16x8 pb[2];
+        const float tm = softmax_max<1, true>(s, t0 + hs * kStepKeys, lim[rb], a.scale_log2, half);
+        softmax_rescale(st.o[rb], m[rb], st.l[rb], tm);
+        softmax_exp<1>(s, pb, m[rb], st.l[rb], a.scale_log2);
+#pragma unroll
+        for (int f = 0; f < 8; ++f)
+          st.o[rb][f & 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(read_v(sV, tl, f), pb[f >> 2], st.o[rb][f & 3],
+                                                                     0, 0, 0);
+      }
+    }
+    lds_barrier();
+  }
+#pragma unroll
+  for (int rb = 0; rb < kPfRB; ++rb) st.nm[rb] = -m[rb];
+}
+
+template <int G, bool PAGED, bool CAUSAL>
+__global__ __launch_bounds__(kPfThreads, 1) void prefill_kernel(const AttnArgs a) {
   constexpr int D = kHeadDim;
   constexpr int TN = kTileKeys;
   constexpr int TM = kPrefillRows / G;
   static_assert(TM >= 32, "a 32-row block is one head");
-  const int b = it.x;
-  const int qt = it.y;
-  const int tb = it.z & 0xffff;
-  const int te = it.z >> 16;
-  const int part = it.w < 0 ? -1 : it.w * a.num_kv_heads + g;
-  // The work list is trusted only as far as the buffers reach: an entry naming a sequence or
-  // key tiles outside this call (a workspace overwritten by an overlapping call) is skipped.
-  // The hooks run in every case, so the work-group's barriers and claims stay in step.
-  // cuv (lanes 0..3) holds the sequence's bounds, loaded by the caller.
-  const int q0 = __builtin_amdgcn_readlane(cuv, 0);
-  const int Lq = __builtin_amdgcn_readlane(cuv, 1) - q0;
-  const int k0 = __builtin_amdgcn_readlane(cuv, 2);
-  const int Lk = min(__builtin_amdgcn_readlane(cuv, 3) - k0, a.max_seqlen_k);
-  const int P = Lk - Lq;
-  if (b < 0 || b >= a.num_seqs || Lq <= 0 || tb > te || te > (Lk + TN - 1) / TN) {
-    lds_barrier();
-    after_tiles();
-    after_epilogue();
-    return;
-  }
-  const int tok_begin = qt * TM;
-
-  const int col = lane & 31;   // MFMA column = this lane's query row inside a block
-  const int half = lane >> 5;
-  int row[kRowBlocks], h[kRowBlocks], tok[kRowBlocks], lim[kRowBlocks], lim_lo[kRowBlocks], lim_hi[kRowBlocks];
-#pragma unroll
-  for (int rb = 0; rb < kRowBlocks; ++rb) {
-    const int r0 = (wave * kRowBlocks + rb) * 32;  // first row of the block: 32 tokens of one head
-    row[rb] = r0 + col;
-    h[rb] = g * G + row[rb] / TM;
-    tok[rb] = tok_begin + row[rb] % TM;
-    lim[rb] = CAUSAL ? min(Lk - 1, tok[rb] + P) : Lk - 1;  // last key this row sees
-    const int blo = tok_begin + r0 % TM;
-    lim_lo[rb] = CAUSAL ? min(Lk - 1, blo + P) : Lk - 1;       // keys <= lim_lo: seen by all rows
-    lim_hi[rb] = CAUSAL ? min(Lk - 1, blo + 31 + P) : Lk - 1;  // keys >  lim_hi: seen by none
-  }
-
-  // Q^T B operands: k-block kb covers d in [16 kb, 16 kb + 16); lane holds 8 of them.
-  // Rows past Lq read the last row (finite) and are never stored.
-  bf16x8 qb[kRowBlocks][D / 16];
-#pragma unroll
-  for (int rb = 0; rb < kRowBlocks; ++rb) {
-    const uint16_t* qp = a.q + (int64_t)(q0 + min(tok[rb], Lq - 1)) * a.q_row_stride + h[rb] * D + 8 * half;
-#pragma unroll
-    for (int kb = 0; kb < D / 16; ++kb)
-      qb[rb][kb] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(qp + kb * 16));
-  }
-  f32x16 o[kRowBlocks][4];
-  float m_i[kRowBlocks], l_i[kRowBlocks];
-#pragma unroll
-  for (int rb = 0; rb < kRowBlocks; ++rb) {
-#pragma unroll
-    for (int md = 0; md < 4; ++md)
-#pragma unroll
-      for (int rr = 0; rr < 16; ++rr) o[rb][md][rr] = 0.f;
-    m_i[rb] = -INFINITY;
-    l_i[rb] = 0.f;
-  }
-
-  // Pipeline, one barrier per tile: at step n, tile n + 1 (registers) is written to stage
-  // (n + 1) & 1 and the loads of tile n + 2 go out into the same registers, tile n is computed
-  // from stage n & 1, and the barrier publishes tile n + 1.
-  const int ntiles = te - tb;
-  const int tbase = tb * TN;
-  const LoadLanes ll = load_lanes(a, wave, lane, kTileKeys);
-  const TileLanes tl = tile_lanes(lane);
-  KvRegs R;
-  // The tile loop is entered only from the path that stored tile 0, whose register wait also
-  // covers the Q loads issued before it. (With a path around that store into the loop, the
-  // compiler's wait counting assumed the Q loads could still be in flight in every iteration
-  // and made each k-block's QK MFMA wait for the global loads issued before it -- tile n + 2's
-  // staging loads -- exposing their latency in every tile.)
-  if (ntiles <= 0) lds_barrier();
-  else {
-  load_tile_regs<PAGED>(a, b, k0, Lk, g, bt_lane, wave, lane, tbase, ll, R);
-  store_tile_lds(R, KS[0], VS[0], wave, lane);
-  if (ntiles > 1) load_tile_regs<PAGED>(a, b, k0, Lk, g, bt_lane, wave, lane, tbase + TN, ll, R);
-  lds_barrier();
-  for (int n0 = 0; n0 < ntiles; n0 += 2) {
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int n = n0 + s;
-      if (n >= ntiles) break;
-      if (n == ntiles - 1) last_step();
-      const int t0 = tbase + n * TN;
-      // tile n + 1 (loaded during tile n - 1) goes to the other stage -- last read at step
-      // n - 1, before the previous barrier -- and its registers take tile n + 2's loads: one
-      // set of staging registers (a second set, holding tile n + 2 while tile n + 1 waited to
-      // be stored after tile n, took the kernel to 256 VGPRs with spills; 2.4% slower)
-      if (n + 1 < ntiles) {
-        store_tile_lds(R, KS[s ^ 1], VS[s ^ 1], wave, lane);
-        if (n + 2 < ntiles) load_tile_regs<PAGED>(a, b, k0, Lk, g, bt_lane, wave, lane, t0 + 2 * TN, ll, R);
-      }
-      bool any = false, full[kRowBlocks];
-#pragma unroll
-      for (int rb = 0; rb < kRowBlocks; ++rb) {
-        any |= t0 <= lim_hi[rb];
-        full[rb] = t0 + TN - 1 <= lim_lo[rb];
-      }
-      if (any) compute_tile(KS[s], VS[s], tl, qb, o, m_i, l_i, t0, lim, full, a.scale_log2, lane);
-      lds_barrier();
-    }
-  }
-  }
-
-  after_tiles();
-  // Epilogue: O^T element rr of d-block md is d = 32 md + 8 (rr >> 2) + 4 half + (rr & 3).
-#pragma unroll
-  for (int rb = 0; rb < kRowBlocks; ++rb) {
-    const float l_tot = swap_halves_sum(l_i[rb]);
-    if (tok[rb] >= Lq) continue;
-    if (part < 0) {
-      const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;  // a row that saw no key is written as 0
-      uint16_t* op = a.out + (int64_t)(q0 + tok[rb]) * a.out_row_stride + h[rb] * D + 4 * half;
-#pragma unroll
-      for (int md = 0; md < 4; ++md)
-#pragma unroll
-        for (int gq = 0; gq < 4; ++gq) {
-          uint2 w;
-          w.x = pack_bf16x2(o[rb][md][4 * gq] * inv, o[rb][md][4 * gq + 1] * inv);
-          w.y = pack_bf16x2(o[rb][md][4 * gq + 2] * inv, o[rb][md][4 * gq + 3] * inv);
-          *reinterpret_cast<uint2*>(op + md * 32 + 8 * gq) = w;
-        }
-    } else if (part < a.pf_part_cap) {
-      // The split's own output o / l in bf16 -- as precise as an unsplit row's output -- with
-      // (max, sum) in fp32 for the merge. Chunk-major (chunk = 4 dims = d / 4): one store
-      // instruction writes two contiguous 256-byte runs (32 rows x 8 bytes per lane half).
-      const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-      uint16_t* po = a.pf_part_o + (int64_t)part * (32 * kPrefillRows * 4);
-#pragma unroll
-      for (int md = 0; md < 4; ++md)
-#pragma unroll
-        for (int gq = 0; gq < 4; ++gq) {
-          const int chunk = 8 * md + 2 * gq + half;
-          uint2 w;
-          w.x = pack_bf16x2(o[rb][md][4 * gq] * inv, o[rb][md][4 * gq + 1] * inv);
-          w.y = pack_bf16x2(o[rb][md][4 * gq + 2] * inv, o[rb][md][4 * gq + 3] * inv);
-          *reinterpret_cast<uint2*>(po + ((int64_t)chunk * kPrefillRows + row[rb]) * 4) = w;
-        }
-      if (half == 0)
-        *reinterpret_cast<float2*>(a.pf_part_ml + ((int64_t)part * kPrefillRows + row[rb]) * 2) =
-            make_float2(m_i[rb], l_tot);
-    }
-  }
-  after_epilogue();
-}
-
-template <int G, bool PAGED, bool CAUSAL>
-__global__ __launch_bounds__(kPrefillThreads, kWavesPerSimd) void prefill_kernel(const AttnArgs a) {
-  // two stages per operand (constant stage indices put the stage offset in immediates)
-  __shared__ __attribute__((aligned(1024))) char sK[kStages][kTileBytes];
-  __shared__ __attribute__((aligned(1024))) char sV[kStages][kTileBytes];
+  __shared__ __attribute__((aligned(1024))) char smem_[kPfLdsBytes];
   __shared__ int s_item;  // the claimed item index
-  lds_char* KS[kStages];
-  lds_char* VS[kStages];
-#pragma unroll
-  for (int st = 0; st < kStages; ++st) {
-    KS[st] = (lds_char*)sK[st];
-    VS[st] = (lds_char*)sV[st];
-  }
+  __shared__ int s_redo;  // the current item needs a running max
+  lds_char* const smem = (lds_char*)smem_;
+  __attribute__((address_space(3))) int* const redo = (__attribute__((address_space(3))) int*)&s_redo;
 
   const int tid = threadIdx.x;
-  const int lane = tid & (kWave - 1);
+  const int lane_ = tid & (kWave - 1), lane = lane_;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   // Work-groups are dealt to the 8 XCDs round-robin by linear id: this one claims items of
   // sub-queue x = blockIdx mod 8 (items i = 8 j + x, counter x) while it has any, then steals
   // from the others. Wavefront 0 claims; lane 0 owns the atomics.
   const int xcd = blockIdx.x & 7;
   const int num_items = (int)min((int64_t)a.pf_queue[kPrefillQueueMeta], (int64_t)a.pf_item_cap * a.num_kv_heads);
-  // The claim on the own sub-queue goes out when the current item starts its last key tile,
-  // so the atomic overlaps that tile and the work-group holds no item it cannot start yet
-  // (items are long: a claim made earlier would hold one back from idle work-groups at the
-  // end). `pend` is that atomic's result (lane 0).
   bool own = true;
-  int pend = 0;
+  int pend = 0;  // lane 0 of wavefront 0: the claim's result
   const auto claim_issue = [&]() {
-    if (wave == 0 && own && lane == 0) pend = atomicAdd(&a.pf_queue[xcd * kPrefillQueueStride], 1);
+    if (wave == 0 && own && lane == 0) {
+      // the address as a per-lane value keeps the compiler from combining the wavefront's lanes
+      // and waiting for the result here
+      int z = 0;
+      asm volatile("" : "+v"(z));
+      pend = atomicAdd(&a.pf_queue[xcd * kPrefillQueueStride + z], 1);
+    }
   };
   // Wavefront 0: the claimed index, or -1 once every sub-queue is exhausted. Stealing reads
   // the other seven counters at once (lanes 0..6) and takes from the first sub-queue after
@@ -762,75 +1018,403 @@ __global__ __launch_bounds__(kPrefillThreads, kWavesPerSimd) void prefill_kernel
       if (cand < num_items) return (int)cand;
     }
   };
-  if (wave == 0) {
-    claim_issue();
-    const int c = claim_finish();
-    if (lane == 0) s_item = c;
-  }
-  lds_barrier();
-  // The next item's inputs load in two dependent steps around the current item's epilogue:
-  // its work-list group (lanes 0..3) before the epilogue's stores, then the sequence's
-  // bounds (lanes 0..3: cu_q[b], cu_q[b + 1], cu_k[b], cu_k[b + 1]) and first 64
-  // block-table entries (one per lane: a tile's block id is a readlane, not a dependent
-  // global load) after them.
   const auto load_group = [&](int i) {
     return lane < 4 ? reinterpret_cast<const int*>(a.pf_items)[(int64_t)(i / a.num_kv_heads) * 4 + lane] : 0;
-  };
-  // The work list is trusted only as far as the buffers reach: a group naming a sequence
-  // outside this call (a workspace overwritten by an overlapping call) reads sequence 0's
-  // bounds and is skipped by prefill_item.
-  const auto seq_of = [&](int grpv) {
-    const int b = __builtin_amdgcn_readlane(grpv, 0);
-    return b >= 0 && b < a.num_seqs ? b : 0;
   };
   const auto load_bounds = [&](int b) {
     const int32_t* p = lane < 2 ? a.cu_q + b + lane : a.cu_k + b + (lane - 2);
     return lane < 4 ? *p : 0;
   };
-  const auto load_bt = [&](int b) {
+  const auto load_bt = [&](int b) {  // the first 64 block-table entries, one per lane
     if constexpr (!PAGED) return 0;
     return lane < min(a.bt_stride, kWave) ? a.block_table[(int64_t)b * a.bt_stride + lane] : 0;
   };
-  int idx = __builtin_amdgcn_readfirstlane(s_item);
-  int grpv = 0, cuv = 0, btv = 0;
-  if (idx >= 0) {
-    grpv = load_group(idx);
-    cuv = load_bounds(seq_of(grpv));
-    btv = load_bt(seq_of(grpv));
-  }
-  while (idx >= 0) {
-    int next = -1, next_grpv = 0, next_cuv = 0, next_btv = 0;
-    bool claimed = false;
-    const int grp = idx / a.num_kv_heads;
-    const int4 it = make_int4(__builtin_amdgcn_readlane(grpv, 0), __builtin_amdgcn_readlane(grpv, 1),
-                              __builtin_amdgcn_readlane(grpv, 2), __builtin_amdgcn_readlane(grpv, 3));
-    prefill_item<G, PAGED, CAUSAL>(
-        a, it, idx - grp * a.num_kv_heads, cuv, btv, KS, VS, wave, lane,
-        [&]() {
-          claim_issue();
-          claimed = true;
-        },
-        [&]() {
-          // s_item was last read before this item's first barrier
-          if (wave == 0) {
-            if (!claimed) claim_issue();
-            const int c = claim_finish();
-            if (lane == 0) s_item = c;
+  // The next item's inputs, in three steps over the current item's last tiles, each begun at the
+  // top of a tile and ended at its bottom, so that none of the dependent round trips is waited
+  // out: 0 the claim, published by wavefront 0; 1 the work-list entry; 2 the sequence's bounds
+  // and block-table entries. What is kept between tiles is uniform or has arrived.
+  int next = -1, gv = 0, cv = 0, btn = 0;
+  int4 ng = make_int4(0, 0, 0, 0), nc = make_int4(0, 0, 0, 0);
+  const auto next_begin = [&](int s) {
+    if (s == 0) {
+      claim_issue();
+    } else if (s == 1) {
+      next = __builtin_amdgcn_readfirstlane(s_item);
+      if (next >= 0) gv = load_group(next);
+    } else if (s == 2 && next >= 0) {
+      const int b = ng.x >= 0 && ng.x < a.num_seqs ? ng.x : 0;  // see make_item
+      cv = load_bounds(b);
+      btn = load_bt(b);
+    }
+  };
+  const auto lanes4 = [&](int v) {
+    return make_int4(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 1), __builtin_amdgcn_readlane(v, 2),
+                     __builtin_amdgcn_readlane(v, 3));
+  };
+  const auto next_end = [&](int s) {
+    if (s == 0) {
+      if (wave == 0) {
+        const int c = claim_finish();
+        if (lane == 0) s_item = c;
+      }
+    } else if (s == 1) {
+      if (next >= 0) ng = lanes4(gv);
+    } else if (s == 2 && next >= 0) {
+      nc = lanes4(cv);
+      asm volatile("" : "+v"(btn));
+    }
+  };
+
+  const int col = lane & 31;   // MFMA column = this lane's query row inside a block
+  const int half = lane >> 5;
+  const TileLanes tl = tile_lanes(lane);
+  const int wrow = 4 * kPfLoads * wave * kRowBytes;  // this wavefront's rows of a stage
+  const int lds0 = (int)(uintptr_t)smem;
+
+  // The first item is the work-group's own (item blockIdx): no claim, and its work-list entry
+  // loads with the item count (the list has room for more groups than there are work-groups).
+  next = (int)blockIdx.x;
+  ng = lanes4(load_group(next));
+  if (next >= num_items) return;
+  next_begin(2);
+  next_end(2);
+  PfItem it = make_item(a, next, ng, nc);
+  int btv = btn;
+
+  // The start of an item: its Q operands and its first tiles (K 0, K 1, V 0, K 2) are requested.
+  // V lags K by two tiles: v1 and v2 are the K cursor's last two positions.
+  TileCursor<PAGED> cur;
+  int koff[kPfLoads], voff[kPfLoads];
+  const char *v1, *v2;
+  int vt1, vt2;
+  const auto clamp_k = [&]() {
+    if (cur.t0 + TN > it.Lk)
+      stage_offsets<false>((int)a.k_row_stride, wave, per_item(lane_), it.Lk - 1 - cur.t0, koff);
+  };
+  const auto stage_v = [&](const char* src, int t, int lds) {
+    if (t + TN > it.Lk) stage_offsets<true>((int)a.v_row_stride, wave, per_item(lane_), it.Lk - 1 - t, voff);
+    stage_tile(src, voff, lds);
+  };
+  const auto start_item = [&]() {
+    const int lane = per_item(lane_);
+    // Q rows (row r of the wavefront's 64, 16-byte chunk c in slot c ^ (r & 15), as K tiles are
+    // stored); rows past Lq take the last row (finite) and are never stored.
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int r = 4 * i + (lane >> 4);
+      const int row0 = block_row<G>(wave, i >> 3);
+      const int tok = max(0, min(it.qt * TM + row0 % TM + (r & 31), it.Lq - 1));
+      load_lds16(a.q + (int64_t)(it.q0 + tok) * a.q_row_stride + (it.g * G + row0 / TM) * D + ((lane & 15) ^ (r & 15)) * 8,
+                 lds0 + kLdsQ + wave * 64 * kRowBytes + i * 1024);
+    }
+    const int ntiles = it.te - it.tb, tbase = it.tb * TN;
+    cur.init(a, it.b, it.g, it.k0, tbase, ntiles, btv);
+    if (ntiles <= 0) return;
+    stage_offsets<false>((int)a.k_row_stride, wave, lane, kTileKeys, koff);
+    stage_offsets<true>((int)a.v_row_stride, wave, lane, kTileKeys, voff);
+    clamp_k();
+    stage_tile(cur.k, koff, lds0 + kLdsK0 + wrow);
+  };
+  const auto start_rest = [&]() {
+    const int ntiles = it.te - it.tb, tbase = it.tb * TN;
+    if (ntiles <= 0) return;
+    const char* const vfirst = cur.v;
+    cur.advance(a, it.b, it.g, btv);
+    clamp_k();
+    v1 = cur.v;
+    vt1 = cur.t0;
+    stage_tile(cur.k, koff, lds0 + kLdsK1 + wrow);
+    stage_v(vfirst, tbase, lds0 + kLdsV0 + wrow);
+    cur.advance(a, it.b, it.g, btv);
+    clamp_k();
+    v2 = cur.v;
+    vt2 = cur.t0;
+    stage_tile(cur.k, koff, lds0 + kLdsK2 + wrow);
+    cur.advance(a, it.b, it.g, btv);
+    clamp_k();
+  };
+  start_item();
+  start_rest();
+
+  for (;;) {
+    PfState st;
+    const int ntiles = it.te - it.tb, tbase = it.tb * TN;
+    const int P = it.Lk - it.Lq;
+    int lim[kPfRB];
+    int lim_lo = 0x7fffffff, lim_hi = -1;  // keys <= lim_lo: seen by all the wavefront's rows, > lim_hi: by none
+#pragma unroll
+    for (int rb = 0; rb < kPfRB; ++rb) {
+      const int r0 = block_row<G>(wave, rb);  // 32 tokens of one head
+      const int blo = it.qt * TM + r0 % TM;
+      // last key of the item this row sees
+      lim[rb] = min(it.te * TN, CAUSAL ? min(it.Lk, blo + col + P + 1) : it.Lk) - 1;
+      lim_lo = min(lim_lo, CAUSAL ? min(it.Lk - 1, blo + P) : it.Lk - 1);
+      lim_hi = max(lim_hi, CAUSAL ? min(it.Lk - 1, blo + 31 + P) : it.Lk - 1);
+      st.nm[rb] = 0.f;
+      st.l[rb] = 0.f;
+    }
+    const auto clear_o = [&]() {
+#pragma unroll
+      for (int rb = 0; rb < kPfRB; ++rb)
+#pragma unroll
+        for (int md = 0; md < 4; ++md) {
+          const float zero = __int_as_float(per_item(0));
+#pragma unroll
+          for (int rr = 0; rr < 16; ++rr) st.o[rb][md][rr] = zero;
+          asm volatile("" : "+a"(st.o[rb][md]));
+        }
+    };
+    // steps (32 keys) this wavefront's rows see
+    const int nw = min(2 * ntiles, (lim_hi - tbase + kStepKeys) >> 5);
+
+    // everything start_item requested is here; Q^T B operands: k-block kb covers d in
+    // [16 kb, 16 kb + 16), a lane holds 8 of them
+    wait_vm<0>();
+    const int qrow = per_item(kLdsQ + wave * 64 * kRowBytes);
+#pragma unroll
+    for (int rb = 0; rb < kPfRB; ++rb)
+#pragma unroll
+      for (int kb = 0; kb < D / 16; ++kb)
+        st.q[rb][kb] = read_k(smem + qrow + rb * 32 * kRowBytes, tl, kb);
+#pragma unroll
+    for (int kb = 0; kb < D / 16; ++kb) {
+      asm volatile("" : "+v"(st.q[0][kb]));
+      asm volatile("" : "+a"(st.q[1][kb]));
+    }
+    next = -1;
+    if (ntiles < 2) {  // no tile to put the claim in
+      next_begin(0);
+      next_end(0);
+    }
+    lds_barrier();
+    if (threadIdx.x == 0) *redo = 0;  // last read before this barrier, next written after a later one
+    if (ntiles <= 0) {
+      next_begin(1);
+      next_end(1);
+      next_begin(2);
+      next_end(2);
+      clear_o();
+    } else {
+      clear_o();
+      int k0s = kLdsK0, k1s = kLdsK1, k2s = kLdsK2, k3s = kLdsK3;  // K tiles n .. n + 3
+      int v1s = kLdsV2, v0s = kLdsV0, vns = kLdsV1;                // V tiles n - 1 .. n + 1
+      // Body n: loads of K tile n + 3 and V tile n + 1; K tile n + 2 and V tile n land by its end.
+      const auto stage = [&](int n) {
+        if (n + 1 < ntiles) stage_v(v1, vt1, lds0 + vns + wrow);
+        v1 = v2;
+        vt1 = vt2;
+        v2 = cur.v;
+        vt2 = cur.t0;
+        if (n + 3 < ntiles) stage_tile(cur.k, koff, lds0 + k3s + wrow);
+        cur.advance(a, it.b, it.g, btv);
+        clamp_k();
+        next_begin(n + 2 - ntiles);
+      };
+      const auto rotate = [&]() {
+        const int k = k0s;
+        k0s = k1s;
+        k1s = k2s;
+        k2s = k3s;
+        k3s = k;
+        const int v = v1s;
+        v1s = v0s;
+        v0s = vns;
+        vns = v;
+      };
+      const auto finish = [&](int n) {
+        next_end(n + 2 - ntiles);
+        if (n == ntiles) return;
+        if (n + 3 < ntiles)
+          wait_vm<8>();
+        else if (n + 1 < ntiles)
+          wait_vm<4>();
+        else
+          wait_vm<0>();
+        lds_barrier();
+        rotate();
+      };
+      // body 0: the scores of steps 0 and 1, the first softmax
+      stage(0);
+      if (nw > 0) {
+bf16x8 k[16];
+#pragma unroll
+        for (int j = 0; j < kPfAhead; ++j) k[j] = read_k(smem + k0s, tl, j);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          const int f = j + kPfAhead;
+          if (f < 16)
+            k[f] = read_k(smem + k0s + (f >> 3) * 32 * kRowBytes, tl, f & 7);
+          else
+            st.kf[f - 16] = read_k(smem + k1s, tl, f - 16);
+#pragma unroll
+          for (int rb = 0; rb < kPfRB; ++rb) mfma_s(st.s[j >> 3][rb], k[j], st.q[rb][j & 7], (j & 7) == 0, rb);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        // the wait states between an MFMA and a VALU read of its result
+        asm volatile("s_nop 15\n\ts_nop 7"
+                     : "+v"(st.s[0][0]), "+v"(st.s[0][1]), "+v"(st.s[1][0]), "+v"(st.s[1][1]));
+        softmax_first(st, tbase, lim, a.scale_log2, half);
+      } else {  // not used; defined, so that no register carries the last item's through this one
+#pragma unroll
+        for (int rb = 0; rb < kPfRB; ++rb) {
+#pragma unroll
+          for (int rr = 0; rr < 16; ++rr) st.s[0][rb][rr] = st.s[1][rb][rr] = 0.f;
+          st.p[0][rb][0] = st.p[0][rb][1] = u32x4{0, 0, 0, 0};
+        }
+#pragma unroll
+        for (int j = 0; j < kPfAhead; ++j) st.kf[j] = st.q[0][0];
+      }
+      finish(0);
+      int t0 = tbase + kStepKeys;  // first key of step 2n - 1
+      int n = 1;
+      // what the allocator put aside over body 0 comes back before the loop, not in it (its waits
+      // would count the loop's own loads)
+#pragma unroll
+      for (int rb = 0; rb < kPfRB; ++rb)
+        asm volatile("" : "+v"(st.s[1][rb]), "+v"(st.p[0][rb][0]), "+v"(st.p[0][rb][1]), "+v"(st.nm[rb]), "+v"(st.l[rb]));
+#pragma unroll 1
+      for (; t0 + TN - 1 <= lim_lo && n + 4 < ntiles; ++n, t0 += TN) {
+        const lds_char* const ks = smem + k0s;
+        const lds_char* const vs = smem + v1s;
+        pf_iteration<1, false, true>(st, ks, ks + 32 * kRowBytes, vs, tl, t0, lim, a.scale_log2, half, v1, voff,
+                                     lds0 + vns + wrow);
+        pf_iteration<0, false, true>(st, ks + 32 * kRowBytes, smem + k1s, vs + 32 * kRowBytes, tl, t0 + kStepKeys, lim,
+                                     a.scale_log2, half, cur.k, koff, lds0 + k3s + wrow);
+        v1 = v2;
+        v2 = cur.v;
+        cur.step(a, it.b, it.g, btv);
+        wait_vm<8>();
+        lds_barrier();
+        rotate();
+      }
+      vt2 = cur.t0 - TN;
+      vt1 = vt2 - TN;
+      clamp_k();
+#pragma unroll 1
+      for (; t0 + TN - 1 <= lim_lo && n < ntiles; ++n, t0 += TN) {
+        stage(n);
+        const lds_char* const ks = smem + k0s;
+        const lds_char* const vs = smem + v1s;
+        pf_iteration<1, false, false>(st, ks, ks + 32 * kRowBytes, vs, tl, t0, lim, a.scale_log2, half, nullptr, koff, 0);
+        pf_iteration<0, false, false>(st, ks + 32 * kRowBytes, smem + k1s, vs + 32 * kRowBytes, tl, t0 + kStepKeys,
+                                      lim, a.scale_log2, half, nullptr, koff, 0);
+        finish(n);
+      }
+#pragma unroll 1
+      for (; n <= ntiles; ++n, t0 += TN) {
+        stage(n);
+        if (2 * n - 2 < nw) {
+        const lds_char* const ks = smem + k0s;
+        const lds_char* const vs = smem + v1s;
+        pf_iteration<1, true, false>(st, ks, ks + 32 * kRowBytes, vs, tl, t0, lim, a.scale_log2, half, nullptr, koff, 0);
+        pf_iteration<0, true, false>(st, ks + 32 * kRowBytes, smem + k1s, vs + 32 * kRowBytes, tl, t0 + kStepKeys, lim,
+                                     a.scale_log2, half, nullptr, koff, 0);
+        }
+        finish(n);
+      }
+    }
+    // The sum shows whether the item's reference held: a row whose scores rose beyond the headroom
+    // (or that overflowed on the way), or whose scores all lie far below the first step's, has the
+    // whole item done again with a running max.
+    float l_tot[kPfRB];
+    bool bad = false;
+#pragma unroll
+    for (int rb = 0; rb < kPfRB; ++rb) {
+      l_tot[rb] = swap_halves_sum(st.l[rb]);
+      bad |= !(l_tot[rb] <= kSumLimit) || (l_tot[rb] == 0.f && lim[rb] >= tbase);
+    }
+    if (ntiles > 0 && __builtin_amdgcn_ballot_w64(bad) != 0 && lane == 0) *redo = 1;
+    lds_barrier();  // every wavefront is done with the item's tiles
+    if (__builtin_expect(ntiles > 0 && __builtin_amdgcn_readfirstlane(*redo) != 0, 0)) {
+      prefill_item_safe<G, PAGED>(a, st, it, btv, lim, smem, wave, per_item(lane_));
+#pragma unroll
+      for (int rb = 0; rb < kPfRB; ++rb) l_tot[rb] = swap_halves_sum(st.l[rb]);
+    }
+    // the next item's first loads go out before this one's results are written
+    const PfItem done = it;
+    if (next >= 0) {
+      it = make_item(a, next, ng, nc);
+      btv = btn;
+      start_item();
+    }
+    // O^T element rr of d-block md is d = 32 md + 8 (rr >> 2) + 4 half + (rr & 3).
+    const int lane = per_item(lane_), col = lane & 31, half = lane >> 5;
+    float inv[kPfRB];
+#pragma unroll
+    for (int rb = 0; rb < kPfRB; ++rb) {
+      inv[rb] = l_tot[rb] > 0.f ? 1.f / l_tot[rb] : 0.f;  // a row that saw no key is written as 0
+#pragma unroll
+      for (int md = 0; md < 4; ++md) asm volatile("" : "+a"(st.o[rb][md]));
+    }
+    if (done.part < 0) {
+      // Through LDS, so that a store covers 128 consecutive bytes of a row (straight from the
+      // accumulators it would cover 16): 64 dims of a row block in 4 KiB, 16-byte chunk c of row r
+      // in slot c ^ (r & 7). The four pieces take this wavefront's rows of the stages that its
+      // second batch of loads fills, which goes out after they are read.
+      const auto piece = [&](int p) { return smem + (p == 0 ? kLdsO : p == 1 ? kLdsK1 : p == 2 ? kLdsK2 : kLdsV0) + wrow; };
+#pragma unroll
+      for (int p = 0; p < 4; ++p)
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+          const f32x16& o = st.o[p >> 1][2 * (p & 1) + (c >> 2)];
+          const float iv = inv[p >> 1];
+          u32x2 w;
+          w[0] = pack_bf16x2(o[4 * (c & 3)] * iv, o[4 * (c & 3) + 1] * iv);
+          w[1] = pack_bf16x2(o[4 * (c & 3) + 2] * iv, o[4 * (c & 3) + 3] * iv);
+          *reinterpret_cast<__attribute__((address_space(3))) u32x2*>(piece(p) + col * 128 + ((c ^ (col & 7)) << 4) +
+                                                                      half * 8) = w;
+        }
+      u32x4 w[4][4];
+#pragma unroll
+      for (int p = 0; p < 4; ++p)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int r = 8 * i + (lane >> 3);
+          w[p][i] = *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>(
+              piece(p) + r * 128 + (((lane & 7) ^ (r & 7)) << 4));
+        }
+#pragma unroll
+      for (int p = 0; p < 4; ++p)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(w[p][i]));
+      if (next >= 0) start_rest();
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        const int row0 = block_row<G>(wave, p >> 1);
+        const int tok0 = done.qt * TM + row0 % TM + (lane >> 3);
+        uint16_t* op = a.out + (int64_t)(done.q0 + tok0) * a.out_row_stride + (done.g * G + row0 / TM) * D +
+                       64 * (p & 1) + 8 * (lane & 7);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (tok0 + 8 * i < done.Lq) *reinterpret_cast<u32x4*>(op + 8 * i * a.out_row_stride) = w[p][i];
+      }
+    } else {
+      if (next >= 0) start_rest();
+#pragma unroll
+      for (int rb = 0; rb < kPfRB; ++rb) {
+        const int row = block_row<G>(wave, rb) + col;
+        const int tok = done.qt * TM + row % TM;
+        if (done.part >= a.pf_part_cap || tok >= done.Lq) continue;
+        // The split's own output o / l in bf16 -- as precise as an unsplit row's output -- with
+        // (max, sum) in fp32 for the merge. Chunk-major (chunk = 4 dims = d / 4): one store
+        // instruction writes two contiguous 256-byte runs (32 rows x 8 bytes per lane half).
+        uint16_t* po = a.pf_part_o + (int64_t)done.part * (32 * kPrefillRows * 4);
+#pragma unroll
+        for (int md = 0; md < 4; ++md)
+#pragma unroll
+          for (int gq = 0; gq < 4; ++gq) {
+            const int chunk = 8 * md + 2 * gq + half;
+            uint2 w;
+            w.x = pack_bf16x2(st.o[rb][md][4 * gq] * inv[rb], st.o[rb][md][4 * gq + 1] * inv[rb]);
+            w.y = pack_bf16x2(st.o[rb][md][4 * gq + 2] * inv[rb], st.o[rb][md][4 * gq + 3] * inv[rb]);
+            *reinterpret_cast<uint2*>(po + ((int64_t)chunk * kPrefillRows + row) * 4) = w;
           }
-          lds_barrier();
-          next = __builtin_amdgcn_readfirstlane(s_item);
-          if (next >= 0) next_grpv = load_group(next);
-        },
-        [&]() {
-          if (next >= 0) {
-            next_cuv = load_bounds(seq_of(next_grpv));
-            next_btv = load_bt(seq_of(next_grpv));
-          }
-        });
-    idx = next;
-    grpv = next_grpv;
-    cuv = next_cuv;
-    btv = next_btv;
+        if (half == 0)
+          *reinterpret_cast<float2*>(a.pf_part_ml + ((int64_t)done.part * kPrefillRows + row) * 2) =
+              make_float2(l_tot[rb] > 0.f ? -st.nm[rb] : -INFINITY, l_tot[rb]);
+      }
+    }
+    if (next < 0) return;
   }
 }
 
@@ -1213,7 +1797,7 @@ int device_prefill_slots() {
 template <int G, bool PAGED, bool CAUSAL>
 hipError_t launch_prefill_gpc(const AttnArgs& a, hipStream_t stream) {
   hipLaunchKernelGGL((prefill_plan_kernel<G, CAUSAL>), dim3(1), dim3(kPlanThreads), 0, stream, a);
-  hipLaunchKernelGGL((prefill_kernel<G, PAGED, CAUSAL>), dim3(a.pf_slots), dim3(kPrefillThreads), 0, stream, a);
+  hipLaunchKernelGGL((prefill_kernel<G, PAGED, CAUSAL>), dim3(a.pf_slots), dim3(kPfThreads), 0, stream, a);
   hipLaunchKernelGGL((prefill_merge_kernel<G>), dim3(kMergeGroups), dim3(kMergeThreads), 0, stream, a);
   return hipGetLastError();
 }

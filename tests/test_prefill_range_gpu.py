@@ -1,0 +1,80 @@
+"""Chunked prefill and dense prompts whose scores leave the range of the item's first reference:
+rows whose later keys score hundreds above the first 32, far below them, or both, with overflow to
+infinity on the way. The softmax is then close to one-hot, and the oracle (fp32) gives it."""
+import pytest
+import torch
+
+import oracle
+import pagedkv
+from paged_helpers import assert_close_bf16
+
+pytestmark = pytest.mark.gpu
+D = 128
+
+
+def _batch(seqs, hq, hkv, steps, seed):
+    """q and k whose products follow `steps`: key t of every sequence scores 16 steps(t) D^-0.5 more
+    than small noise (exact in bf16 for whole steps up to 256)."""
+    g = torch.Generator().manual_seed(seed)
+    nq, nk = sum(q for q, _ in seqs), sum(k for _, k in seqs)
+    q = 0.25 * torch.randn(nq, hq, D, generator=g)
+    k = 0.25 * torch.randn(nk, hkv, D, generator=g)
+    q[..., 0] = 16.0
+    k[..., 0] = torch.cat([torch.tensor([float(steps(t, n)) for t in range(n)]) for _, n in seqs])[:, None]
+    v = torch.randn(nk, hkv, D, generator=g)
+    return (x.to(torch.bfloat16) for x in (q, k, v))
+
+
+STEPS = {
+    "jump": lambda t, n: 150 if t >= 40 else 0,                 # 212 nats above the first keys
+    "late": lambda t, n: 100 if t == n - 1 else 0,              # one key, at the end
+    "ramp": lambda t, n: min(240, t // 8),                      # up to 339 nats, step by step
+    "fall": lambda t, n: -200 if t >= 32 else 0,                # everything after the first step vanishes
+    "low": lambda t, n: -250 if t < 64 else 0,                  # the first tile vanishes
+    "inside": lambda t, n: 50 if t % 96 == 70 else 0,           # 71 nats: inside the headroom
+}
+
+
+@pytest.mark.parametrize("steps", list(STEPS))
+@pytest.mark.parametrize("hq,hkv", [(16, 8), (4, 4), (8, 1)])
+@pytest.mark.parametrize("paged", [True, False])
+def test_scores_beyond_the_first_reference(gpu, steps, hq, hkv, paged):
+    seqs = [(130, 700), (2, 65), (33, 2000), (257, 257)] if paged else [(130, 130), (2, 2), (600, 600), (65, 65)]
+    print(f"[prefill-range] {steps} hq={hq} hkv={hkv} paged={paged}", flush=True)
+    q, k, v = _batch(seqs, hq, hkv, STEPS[steps], 7)
+    cu_q = torch.tensor([0] + list(torch.tensor([a for a, _ in seqs]).cumsum(0)), dtype=torch.int32)
+    cu_k = torch.tensor([0] + list(torch.tensor([b for _, b in seqs]).cumsum(0)), dtype=torch.int32)
+    bt = None
+    kc, vc = k, v
+    if paged:
+        bs, width = 64, max((n + 63) // 64 for _, n in seqs)
+        blocks = sum((n + bs - 1) // bs for _, n in seqs)
+        order = torch.randperm(blocks, generator=torch.Generator().manual_seed(1)).tolist()
+        kc, vc = (torch.zeros(blocks, bs, hkv, D, dtype=torch.bfloat16) for _ in range(2))
+        bt = torch.full((len(seqs), width), -1, dtype=torch.int32)
+        for b, (_, n) in enumerate(seqs):
+            for j in range((n + bs - 1) // bs):
+                blk, lo, m = order.pop(), int(cu_k[b]) + j * bs, min(bs, n - j * bs)
+                bt[b, j] = blk
+                kc[blk, :m], vc[blk, :m] = k[lo:lo + m], v[lo:lo + m]
+    want = oracle.varlen_attention(q, kc, vc, cu_q, cu_k, D ** -0.5, True, bt)
+    dev = [None if x is None else x.to(gpu) for x in (q, kc, vc, cu_q, cu_k, bt)]
+    out = pagedkv.varlen_attention(dev[0], dev[1], dev[2], dev[3], dev[4], max(a for a, _ in seqs),
+                                   max(b for _, b in seqs), D ** -0.5, True, dev[5], cached_prefix_keys=0)
+    torch.cuda.synchronize()
+    assert_close_bf16(out, want, f"{steps} paged={paged}")
+
+
+@pytest.mark.parametrize("tail", [1, 31, 32, 33, 63, 64, 65, 127, 128, 129, 191, 192, 193, 320])
+def test_step_and_tile_edges(gpu, tail):
+    """Key counts around the 32-key steps, the tiles and the depth of the tile pipeline."""
+    seqs = [(max(2, tail), tail + 1), (2, tail + 1), (64, tail + 64), (127, tail + 130)]
+    print(f"[prefill-range] edges tail={tail}", flush=True)
+    q, k, v = _batch(seqs, 8, 4, lambda t, n: 0, tail)
+    cu_q = torch.tensor([0] + list(torch.tensor([a for a, _ in seqs]).cumsum(0)), dtype=torch.int32)
+    cu_k = torch.tensor([0] + list(torch.tensor([b for _, b in seqs]).cumsum(0)), dtype=torch.int32)
+    want = oracle.varlen_attention(q, k, v, cu_q, cu_k, D ** -0.5, True, None)
+    out = pagedkv.varlen_attention(q.to(gpu), k.to(gpu), v.to(gpu), cu_q.to(gpu), cu_k.to(gpu),
+                                   max(a for a, _ in seqs), max(b for _, b in seqs), D ** -0.5, True, None)
+    torch.cuda.synchronize()
+    assert_close_bf16(out, want, f"tail {tail}")
