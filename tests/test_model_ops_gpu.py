@@ -105,3 +105,18 @@ def test_lm_head_greedy_one_hot_ties(gpu):
     h[2, :8] = -1.0
     got = pagedkv.lm_head_greedy(h.to(torch.bfloat16).to(gpu), w.to(torch.bfloat16).to(gpu))
     assert got.tolist() == [5, 1, 0]
+
+
+@pytest.mark.parametrize("hidden", [128, 384, 1024])
+@pytest.mark.parametrize("rows,vocab", [(1, 31), (31, 33), (32, 4096), (33, 8191), (64, 8193), (65, 16385), (97, 600),
+                                        (128, 20000), (129, 2048)])
+def test_lm_head_greedy_row_blocks_and_k_slices(gpu, rows, vocab, hidden):
+    """Every count of 32-row blocks, fewer K slices than wavefronts, vocabularies that end inside a
+    tile or hold fewer tiles than there are work-groups, and strided rows."""
+    print(f"[lm-head] rows={rows} vocab={vocab} hidden={hidden}", flush=True)
+    w = _rand((vocab, hidden + 64), 21, 0.02)[:, :hidden]
+    h = _rand((rows, hidden + 8), 22 + rows)[:, :hidden]
+    wd = w.to(gpu) if w.is_contiguous() else torch.empty(vocab, hidden + 64, dtype=torch.bfloat16, device=gpu)[:, :hidden].copy_(w)
+    hd = torch.empty(rows, hidden + 8, dtype=torch.bfloat16, device=gpu)[:, :hidden].copy_(h)
+    got = pagedkv.lm_head_greedy(hd, wd)
+    _greedy_check(got, h.contiguous(), w.contiguous())
