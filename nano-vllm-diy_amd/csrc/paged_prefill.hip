@@ -76,9 +76,11 @@ constexpr int kMergeLoads = PK_MERGE_LOADS;  // merge: splits whose outputs load
 #ifndef PK_PREFILL_BUCKETS
 #define PK_PREFILL_BUCKETS 8
 #endif
-// length buckets of the work list (longest first): 4 -> 8 took the dense prompts 144.4 -> 141.6 us
-// and the long chunks 605 -> 594 us; 16 gave 146.3 and 594
+// Length buckets of the work list (longest first). prefill_kernel: 4 -> 8 took the dense prompts
+// 144.4 -> 141.6 us and the long chunks 605 -> 594 us, 16 gave 146.3 and 594; prefill_w8_kernel
+// keeps 4 (8: 31 prompts of 512 114.2 -> 118.9 us, 15 chunks of 100 over 4096 keys 117.5 -> 119.9).
 constexpr int kBuckets = PK_PREFILL_BUCKETS;
+constexpr int kSmallBuckets = 4;
 constexpr float kLazyLog2 = 8.f;       // reference max moves only when exceeded by 2^8
 
 typedef short v4i16 __attribute__((ext_vector_type(4)));
@@ -167,6 +169,27 @@ __device__ __forceinline__ void load_rows(const uint16_t* kbase, const uint16_t*
     R.k[i] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(kbase) + l.k[i]);
     R.v[i] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(vbase) + l.v[i]);
   }
+}
+
+template <bool PAGED>
+__device__ __forceinline__ void load_tile_regs(const AttnArgs& a, int b, int k0, int Lk, int g, int bt_lane, int wave,
+                                               int lane, int t0, const LoadLanes& full_lanes, KvRegs& R) {
+  const uint16_t* kbase;
+  const uint16_t* vbase;
+  if constexpr (PAGED) {
+    const int j = t0 / a.block_size;  // block_size % 64 == 0: the tile sits inside one block
+    const int blk = j < kWave ? __builtin_amdgcn_readlane(bt_lane, j)
+                              : __builtin_amdgcn_readfirstlane(a.block_table[(int64_t)b * a.bt_stride + j]);
+    const int off = t0 % a.block_size;
+    kbase = a.k + (int64_t)blk * a.k_block_stride + (int64_t)off * a.k_row_stride;
+    vbase = a.v + (int64_t)blk * a.v_block_stride + (int64_t)off * a.v_row_stride;
+  } else {
+    kbase = a.k + (int64_t)(k0 + t0) * a.k_row_stride;
+    vbase = a.v + (int64_t)(k0 + t0) * a.v_row_stride;
+  }
+  kbase += g * kHeadDim;
+  vbase += g * kHeadDim;
+  load_rows(kbase, vbase, (t0 + kTileKeys <= Lk) ? full_lanes : load_lanes(a, wave, lane, Lk - 1 - t0), R);
 }
 
 __device__ __forceinline__ void store_tile_lds(const KvRegs& R, lds_char* kdst, lds_char* vdst, int wave, int lane) {
@@ -404,12 +427,12 @@ __device__ __forceinline__ int unit_tiles(const SeqDims& d, int qt) {
 __device__ __forceinline__ int unit_splits(int t, int T) { return t > T ? (t + T - 1) / T : 1; }
 __device__ __forceinline__ int split_begin(int t, int n, int s) { return (int)((unsigned)(t * s) / (unsigned)n); }
 
-// Length bucket of a group of t tiles (0 = longest) for split size T.
-__device__ __forceinline__ int length_bucket(int t, int T) {
-  int j = 0;  // the largest j < kBuckets with t kBuckets > j T (compares, no division)
+// Length bucket of a group of t tiles (0 = longest) of n buckets for split size T.
+__device__ __forceinline__ int length_bucket(int t, int T, int n) {
+  int j = 0;  // the largest j < n with t n > j T (compares, no division)
 #pragma unroll
-  for (int i = 1; i < kBuckets; ++i) j = t * kBuckets > i * T ? i : j;
-  return kBuckets - 1 - j;
+  for (int i = 1; i < kBuckets; ++i) j = i < n && t * n > i * T ? i : j;
+  return n - 1 - j;
 }
 
 // Work list. Waves take sequences in turn and lanes take a sequence's query tiles, so a
@@ -488,7 +511,7 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const AttnAr
       const int t = unit_tiles<TM, CAUSAL>(d, qt);
       const int n = unit_splits(t, T);
       for (int sp = 0; sp < n; ++sp)
-        atomicAdd(&cur[length_bucket(split_begin(t, n, sp + 1) - split_begin(t, n, sp), T)], 1);
+        atomicAdd(&cur[length_bucket(split_begin(t, n, sp + 1) - split_begin(t, n, sp), T, a.pf_buckets)], 1);
     }
   }
   __syncthreads();
@@ -515,7 +538,7 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const AttnAr
       for (int sp = 0; sp < n; ++sp) {
         const int tb = split_begin(t, n, sp);
         const int te = split_begin(t, n, sp + 1);
-        const int k = length_bucket(te - tb, T);
+        const int k = length_bucket(te - tb, T, a.pf_buckets);
         const int grp = start[k] + atomicAdd(&cur[k], 1);
         if (grp < a.pf_item_cap) a.pf_items[grp] = make_int4(b, qt, tb | (te << 16), n > 1 ? pg + sp : -1);
       }
@@ -534,6 +557,300 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const AttnAr
     a.pf_queue[kPrefillQueueMeta] = (int)(min((int64_t)tot, (int64_t)a.pf_item_cap) * hkv);
     a.pf_queue[kPrefillQueueMeta + 1] = (int)(min((int64_t)cur[kBuckets + 1], (int64_t)a.pf_merge_cap) * hkv);
     a.pf_queue[kPrefillQueueMeta + 2] = T;
+  }
+}
+
+// ---- Small calls ---------------------------------------------------------------------------
+// Eight wavefronts of one row block each (two per SIMD) in phases QK - softmax - PV per 64-key
+// tile, K and V through registers into two LDS stages. Its tile takes half as long again as
+// prefill_kernel's, but an item starts sooner (no pipeline to fill, a third of the code to fetch
+// into a cold instruction cache), which decides where a work-group has one or two short items:
+// one item of 7 tiles per work-group 36.7 against 40.9 us a call, 15 chunks of 100 over 2048
+// keys 74.5 against 81.0. prefill_kernel is ahead from about 36 tiles per work-group (see
+// launch_prefill_gpc).
+constexpr int kW8Stages = 2;             // K and V LDS stages
+
+// One work item: kv head g of group `it` = (sequence b, query tile qt, key tiles [tb, te),
+// partial group or -1). The caller's hooks run at three points, which the kernel uses to
+// claim and prefetch the next item: last_step when the last key tile starts, after_tiles
+// after the last tile's barrier (before the epilogue), after_epilogue after its stores.
+template <int G, bool PAGED, bool CAUSAL, class LastStep, class AfterTiles, class AfterEpilogue>
+__device__ __forceinline__ void prefill_item_w8(const AttnArgs& a, const int4 it, const int g, const int cuv,
+                                             const int bt_lane, lds_char* const (&KS)[kW8Stages],
+                                             lds_char* const (&VS)[kW8Stages],
+                                             int wave, int lane,
+                                             LastStep&& last_step, AfterTiles&& after_tiles,
+                                             AfterEpilogue&& after_epilogue) {
+  constexpr int D = kHeadDim;
+  constexpr int TN = kTileKeys;
+  constexpr int TM = kPrefillRows / G;
+  static_assert(TM >= 32, "a 32-row block is one head");
+  const int b = it.x;
+  const int qt = it.y;
+  const int tb = it.z & 0xffff;
+  const int te = it.z >> 16;
+  const int part = it.w < 0 ? -1 : it.w * a.num_kv_heads + g;
+  // The work list is trusted only as far as the buffers reach: an entry naming a sequence or
+  // key tiles outside this call (a workspace overwritten by an overlapping call) is skipped.
+  // The hooks run in every case, so the work-group's barriers and claims stay in step.
+  // cuv (lanes 0..3) holds the sequence's bounds, loaded by the caller.
+  const int q0 = __builtin_amdgcn_readlane(cuv, 0);
+  const int Lq = __builtin_amdgcn_readlane(cuv, 1) - q0;
+  const int k0 = __builtin_amdgcn_readlane(cuv, 2);
+  const int Lk = min(__builtin_amdgcn_readlane(cuv, 3) - k0, a.max_seqlen_k);
+  const int P = Lk - Lq;
+  if (b < 0 || b >= a.num_seqs || Lq <= 0 || tb > te || te > (Lk + TN - 1) / TN) {
+    lds_barrier();
+    after_tiles();
+    after_epilogue();
+    return;
+  }
+  const int tok_begin = qt * TM;
+
+  const int col = lane & 31;   // MFMA column = this lane's query row inside a block
+  const int half = lane >> 5;
+  int row[kRowBlocks], h[kRowBlocks], tok[kRowBlocks], lim[kRowBlocks], lim_lo[kRowBlocks], lim_hi[kRowBlocks];
+#pragma unroll
+  for (int rb = 0; rb < kRowBlocks; ++rb) {
+    const int r0 = (wave * kRowBlocks + rb) * 32;  // first row of the block: 32 tokens of one head
+    row[rb] = r0 + col;
+    h[rb] = g * G + row[rb] / TM;
+    tok[rb] = tok_begin + row[rb] % TM;
+    lim[rb] = CAUSAL ? min(Lk - 1, tok[rb] + P) : Lk - 1;  // last key this row sees
+    const int blo = tok_begin + r0 % TM;
+    lim_lo[rb] = CAUSAL ? min(Lk - 1, blo + P) : Lk - 1;       // keys <= lim_lo: seen by all rows
+    lim_hi[rb] = CAUSAL ? min(Lk - 1, blo + 31 + P) : Lk - 1;  // keys >  lim_hi: seen by none
+  }
+
+  // Q^T B operands: k-block kb covers d in [16 kb, 16 kb + 16); lane holds 8 of them.
+  // Rows past Lq read the last row (finite) and are never stored.
+  bf16x8 qb[kRowBlocks][D / 16];
+#pragma unroll
+  for (int rb = 0; rb < kRowBlocks; ++rb) {
+    const uint16_t* qp = a.q + (int64_t)(q0 + min(tok[rb], Lq - 1)) * a.q_row_stride + h[rb] * D + 8 * half;
+#pragma unroll
+    for (int kb = 0; kb < D / 16; ++kb)
+      qb[rb][kb] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(qp + kb * 16));
+  }
+  f32x16 o[kRowBlocks][4];
+  float m_i[kRowBlocks], l_i[kRowBlocks];
+#pragma unroll
+  for (int rb = 0; rb < kRowBlocks; ++rb) {
+#pragma unroll
+    for (int md = 0; md < 4; ++md)
+#pragma unroll
+      for (int rr = 0; rr < 16; ++rr) o[rb][md][rr] = 0.f;
+    m_i[rb] = -INFINITY;
+    l_i[rb] = 0.f;
+  }
+
+  // Pipeline, one barrier per tile: at step n, tile n + 1 (registers) is written to stage
+  // (n + 1) & 1 and the loads of tile n + 2 go out into the same registers, tile n is computed
+  // from stage n & 1, and the barrier publishes tile n + 1.
+  const int ntiles = te - tb;
+  const int tbase = tb * TN;
+  const LoadLanes ll = load_lanes(a, wave, lane, kTileKeys);
+  const TileLanes tl = tile_lanes(lane);
+  KvRegs R;
+  // The tile loop is entered only from the path that stored tile 0, whose register wait also
+  // covers the Q loads issued before it. (With a path around that store into the loop, the
+  // compiler's wait counting assumed the Q loads could still be in flight in every iteration
+  // and made each k-block's QK MFMA wait for the global loads issued before it -- tile n + 2's
+  // staging loads -- exposing their latency in every tile.)
+  if (ntiles <= 0) lds_barrier();
+  else {
+  load_tile_regs<PAGED>(a, b, k0, Lk, g, bt_lane, wave, lane, tbase, ll, R);
+  store_tile_lds(R, KS[0], VS[0], wave, lane);
+  if (ntiles > 1) load_tile_regs<PAGED>(a, b, k0, Lk, g, bt_lane, wave, lane, tbase + TN, ll, R);
+  lds_barrier();
+  for (int n0 = 0; n0 < ntiles; n0 += 2) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int n = n0 + s;
+      if (n >= ntiles) break;
+      if (n == ntiles - 1) last_step();
+      const int t0 = tbase + n * TN;
+      // tile n + 1 (loaded during tile n - 1) goes to the other stage -- last read at step
+      // n - 1, before the previous barrier -- and its registers take tile n + 2's loads: one
+      // set of staging registers (a second set, holding tile n + 2 while tile n + 1 waited to
+      // be stored after tile n, took the kernel to 256 VGPRs with spills; 2.4% slower)
+      if (n + 1 < ntiles) {
+        store_tile_lds(R, KS[s ^ 1], VS[s ^ 1], wave, lane);
+        if (n + 2 < ntiles) load_tile_regs<PAGED>(a, b, k0, Lk, g, bt_lane, wave, lane, t0 + 2 * TN, ll, R);
+      }
+      bool any = false, full[kRowBlocks];
+#pragma unroll
+      for (int rb = 0; rb < kRowBlocks; ++rb) {
+        any |= t0 <= lim_hi[rb];
+        full[rb] = t0 + TN - 1 <= lim_lo[rb];
+      }
+      if (any) compute_tile(KS[s], VS[s], tl, qb, o, m_i, l_i, t0, lim, full, a.scale_log2, lane);
+      lds_barrier();
+    }
+  }
+  }
+
+  after_tiles();
+  // Epilogue: O^T element rr of d-block md is d = 32 md + 8 (rr >> 2) + 4 half + (rr & 3).
+#pragma unroll
+  for (int rb = 0; rb < kRowBlocks; ++rb) {
+    const float l_tot = swap_halves_sum(l_i[rb]);
+    if (tok[rb] >= Lq) continue;
+    if (part < 0) {
+      const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;  // a row that saw no key is written as 0
+      uint16_t* op = a.out + (int64_t)(q0 + tok[rb]) * a.out_row_stride + h[rb] * D + 4 * half;
+#pragma unroll
+      for (int md = 0; md < 4; ++md)
+#pragma unroll
+        for (int gq = 0; gq < 4; ++gq) {
+          uint2 w;
+          w.x = pack_bf16x2(o[rb][md][4 * gq] * inv, o[rb][md][4 * gq + 1] * inv);
+          w.y = pack_bf16x2(o[rb][md][4 * gq + 2] * inv, o[rb][md][4 * gq + 3] * inv);
+          *reinterpret_cast<uint2*>(op + md * 32 + 8 * gq) = w;
+        }
+    } else if (part < a.pf_part_cap) {
+      // The split's own output o / l in bf16 -- as precise as an unsplit row's output -- with
+      // (max, sum) in fp32 for the merge. Chunk-major (chunk = 4 dims = d / 4): one store
+      // instruction writes two contiguous 256-byte runs (32 rows x 8 bytes per lane half).
+      const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+      uint16_t* po = a.pf_part_o + (int64_t)part * (32 * kPrefillRows * 4);
+#pragma unroll
+      for (int md = 0; md < 4; ++md)
+#pragma unroll
+        for (int gq = 0; gq < 4; ++gq) {
+          const int chunk = 8 * md + 2 * gq + half;
+          uint2 w;
+          w.x = pack_bf16x2(o[rb][md][4 * gq] * inv, o[rb][md][4 * gq + 1] * inv);
+          w.y = pack_bf16x2(o[rb][md][4 * gq + 2] * inv, o[rb][md][4 * gq + 3] * inv);
+          *reinterpret_cast<uint2*>(po + ((int64_t)chunk * kPrefillRows + row[rb]) * 4) = w;
+        }
+      if (half == 0)
+        *reinterpret_cast<float2*>(a.pf_part_ml + ((int64_t)part * kPrefillRows + row[rb]) * 2) =
+            make_float2(m_i[rb], l_tot);
+    }
+  }
+  after_epilogue();
+}
+
+template <int G, bool PAGED, bool CAUSAL>
+__global__ __launch_bounds__(kPrefillThreads, kWavesPerSimd) void prefill_w8_kernel(const AttnArgs a) {
+  // two stages per operand (constant stage indices put the stage offset in immediates)
+  __shared__ __attribute__((aligned(1024))) char sK[kW8Stages][kTileBytes];
+  __shared__ __attribute__((aligned(1024))) char sV[kW8Stages][kTileBytes];
+  __shared__ int s_item;  // the claimed item index
+  lds_char* KS[kW8Stages];
+  lds_char* VS[kW8Stages];
+#pragma unroll
+  for (int st = 0; st < kW8Stages; ++st) {
+    KS[st] = (lds_char*)sK[st];
+    VS[st] = (lds_char*)sV[st];
+  }
+
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  // Work-groups are dealt to the 8 XCDs round-robin by linear id: this one claims items of
+  // sub-queue x = blockIdx mod 8 (items i = 8 j + x, counter x) while it has any, then steals
+  // from the others. Wavefront 0 claims; lane 0 owns the atomics.
+  const int xcd = blockIdx.x & 7;
+  const int num_items = (int)min((int64_t)a.pf_queue[kPrefillQueueMeta], (int64_t)a.pf_item_cap * a.num_kv_heads);
+  // The claim on the own sub-queue goes out when the current item starts its last key tile,
+  // so the atomic overlaps that tile and the work-group holds no item it cannot start yet
+  // (items are long: a claim made earlier would hold one back from idle work-groups at the
+  // end). `pend` is that atomic's result (lane 0).
+  bool own = true;
+  int pend = 0;
+  const auto claim_issue = [&]() {
+    if (wave == 0 && own && lane == 0) pend = atomicAdd(&a.pf_queue[xcd * kPrefillQueueStride], 1);
+  };
+  // Wavefront 0: the claimed index, or -1 once every sub-queue is exhausted. Stealing reads
+  // the other seven counters at once (lanes 0..6) and takes from the first sub-queue after
+  // this one that has items left; a claim that lost the race reads again. Counters only
+  // grow, so a stale read never shows a sub-queue exhausted too early.
+  const auto claim_finish = [&]() {
+    if (own) {
+      const int64_t cand = (int64_t)__builtin_amdgcn_readfirstlane(pend) * 8 + xcd;
+      if (cand < num_items) return (int)cand;
+      own = false;
+    }
+    for (;;) {
+      const int q = (xcd + 1 + lane) & 7;
+      const int c = lane < 7 ? __hip_atomic_load(&a.pf_queue[q * kPrefillQueueStride], __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT)
+                             : 0;
+      const uint64_t left = __builtin_amdgcn_ballot_w64(lane < 7 && (int64_t)c * 8 + q < num_items);
+      if (left == 0) return -1;
+      const int qs = (xcd + 1 + __builtin_ctzll(left)) & 7;
+      int r = 0;
+      if (lane == 0) r = atomicAdd(&a.pf_queue[qs * kPrefillQueueStride], 1);
+      const int64_t cand = (int64_t)__builtin_amdgcn_readfirstlane(r) * 8 + qs;
+      if (cand < num_items) return (int)cand;
+    }
+  };
+  // The next item's inputs load in two dependent steps around the current item's epilogue:
+  // its work-list group (lanes 0..3) before the epilogue's stores, then the sequence's
+  // bounds (lanes 0..3: cu_q[b], cu_q[b + 1], cu_k[b], cu_k[b + 1]) and first 64
+  // block-table entries (one per lane: a tile's block id is a readlane, not a dependent
+  // global load) after them.
+  const auto load_group = [&](int i) {
+    return lane < 4 ? reinterpret_cast<const int*>(a.pf_items)[(int64_t)(i / a.num_kv_heads) * 4 + lane] : 0;
+  };
+  // The work list is trusted only as far as the buffers reach: a group naming a sequence
+  // outside this call (a workspace overwritten by an overlapping call) reads sequence 0's
+  // bounds and is skipped by prefill_item.
+  const auto seq_of = [&](int grpv) {
+    const int b = __builtin_amdgcn_readlane(grpv, 0);
+    return b >= 0 && b < a.num_seqs ? b : 0;
+  };
+  const auto load_bounds = [&](int b) {
+    const int32_t* p = lane < 2 ? a.cu_q + b + lane : a.cu_k + b + (lane - 2);
+    return lane < 4 ? *p : 0;
+  };
+  const auto load_bt = [&](int b) {
+    if constexpr (!PAGED) return 0;
+    return lane < min(a.bt_stride, kWave) ? a.block_table[(int64_t)b * a.bt_stride + lane] : 0;
+  };
+  // the first item is the work-group's own (item blockIdx), as in prefill_kernel
+  int idx = (int)blockIdx.x < num_items ? (int)blockIdx.x : -1;
+  int grpv = 0, cuv = 0, btv = 0;
+  if (idx >= 0) {
+    grpv = load_group(idx);
+    cuv = load_bounds(seq_of(grpv));
+    btv = load_bt(seq_of(grpv));
+  }
+  while (idx >= 0) {
+    int next = -1, next_grpv = 0, next_cuv = 0, next_btv = 0;
+    bool claimed = false;
+    const int grp = idx / a.num_kv_heads;
+    const int4 it = make_int4(__builtin_amdgcn_readlane(grpv, 0), __builtin_amdgcn_readlane(grpv, 1),
+                              __builtin_amdgcn_readlane(grpv, 2), __builtin_amdgcn_readlane(grpv, 3));
+    prefill_item_w8<G, PAGED, CAUSAL>(
+        a, it, idx - grp * a.num_kv_heads, cuv, btv, KS, VS, wave, lane,
+        [&]() {
+          claim_issue();
+          claimed = true;
+        },
+        [&]() {
+          // s_item was last read before this item's first barrier
+          if (wave == 0) {
+            if (!claimed) claim_issue();
+            const int c = claim_finish();
+            if (lane == 0) s_item = c;
+          }
+          lds_barrier();
+          next = __builtin_amdgcn_readfirstlane(s_item);
+          if (next >= 0) next_grpv = load_group(next);
+        },
+        [&]() {
+          if (next >= 0) {
+            next_cuv = load_bounds(seq_of(next_grpv));
+            next_btv = load_bt(seq_of(next_grpv));
+          }
+        });
+    idx = next;
+    grpv = next_grpv;
+    cuv = next_cuv;
+    btv = next_btv;
   }
 }
 
@@ -1795,9 +2112,24 @@ int device_prefill_slots() {
 }
 
 template <int G, bool PAGED, bool CAUSAL>
-hipError_t launch_prefill_gpc(const AttnArgs& a, hipStream_t stream) {
+hipError_t launch_prefill_gpc(AttnArgs a, hipStream_t stream) {
+  // Which kernel: the launch bounds' tiles per work-group, if every sequence were as long as they
+  // allow (the lengths are on the device). Uniform batches, w8 kernel against prefill_kernel (us
+  // per call). Paged: 15 tiles 60.8 / 63.0, 16 74.5 / 81.0, 20 81.4 / 81.5 and 79.6 / 81.5, 31
+  // 115.8 / 118.8, 36 114.9 / 111.7, 37 115.2 / 114.3, 48 124.0 / 119.9, 300 619 / 554. Flat (a
+  // prompt's tiles are half the bound): 4 39.7 / 41.1, 8 44.8 / 47.0, 16 103.6 / 104.8, 31 112.9 /
+  // 112.0, 64 108.9 / 104.6, 256 315 / 288. A ragged batch is taken for a larger one: that costs
+  // at most the few us by which the small calls differ.
+  constexpr int kSmallTiles = PAGED ? 36 : 24;
+  const int64_t tiles = (int64_t)a.num_seqs * a.prefill_qtiles * ((a.max_seqlen_k + kTileKeys - 1) / kTileKeys) *
+                        a.num_kv_heads;
+  const bool small = tiles < (int64_t)kSmallTiles * a.pf_slots;
+  a.pf_buckets = small ? kSmallBuckets : kBuckets;
   hipLaunchKernelGGL((prefill_plan_kernel<G, CAUSAL>), dim3(1), dim3(kPlanThreads), 0, stream, a);
-  hipLaunchKernelGGL((prefill_kernel<G, PAGED, CAUSAL>), dim3(a.pf_slots), dim3(kPfThreads), 0, stream, a);
+  if (small)
+    hipLaunchKernelGGL((prefill_w8_kernel<G, PAGED, CAUSAL>), dim3(a.pf_slots), dim3(kPrefillThreads), 0, stream, a);
+  else
+    hipLaunchKernelGGL((prefill_kernel<G, PAGED, CAUSAL>), dim3(a.pf_slots), dim3(kPfThreads), 0, stream, a);
   hipLaunchKernelGGL((prefill_merge_kernel<G>), dim3(kMergeGroups), dim3(kMergeThreads), 0, stream, a);
   return hipGetLastError();
 }

@@ -39,7 +39,9 @@ STEPS = {
 @pytest.mark.parametrize("hq,hkv", [(16, 8), (4, 4), (8, 1)])
 @pytest.mark.parametrize("paged", [True, False])
 def test_scores_beyond_the_first_reference(gpu, steps, hq, hkv, paged):
-    seqs = [(130, 700), (2, 65), (33, 2000), (257, 257)] if paged else [(130, 130), (2, 2), (600, 600), (65, 65)]
+    # bounds of 36 tiles per work-group and more (the pipelined kernel), and with hq, hkv = 8, 1 fewer
+    seqs = [(130, 700), (2, 65), (33, 2000), (257, 257), (1100, 1500), (40, 40)] if paged else \
+        [(130, 130), (2, 2), (1800, 1800), (65, 65), (3, 3), (300, 300)]
     print(f"[prefill-range] {steps} hq={hq} hkv={hkv} paged={paged}", flush=True)
     q, k, v = _batch(seqs, hq, hkv, STEPS[steps], 7)
     cu_q = torch.tensor([0] + list(torch.tensor([a for a, _ in seqs]).cumsum(0)), dtype=torch.int32)
@@ -65,10 +67,14 @@ def test_scores_beyond_the_first_reference(gpu, steps, hq, hkv, paged):
     assert_close_bf16(out, want, f"{steps} paged={paged}")
 
 
+@pytest.mark.parametrize("large", [False, True])
 @pytest.mark.parametrize("tail", [1, 31, 32, 33, 63, 64, 65, 127, 128, 129, 191, 192, 193, 320])
-def test_step_and_tile_edges(gpu, tail):
+def test_step_and_tile_edges(gpu, tail, large):
     """Key counts around the 32-key steps, the tiles and the depth of the tile pipeline."""
+    # the last prompt is there for the launch bounds: enough tiles for the pipelined kernel
     seqs = [(max(2, tail), tail + 1), (2, tail + 1), (64, tail + 64), (127, tail + 130)]
+    if large:
+        seqs.append((2500, 2500))
     print(f"[prefill-range] edges tail={tail}", flush=True)
     q, k, v = _batch(seqs, 8, 4, lambda t, n: 0, tail)
     cu_q = torch.tensor([0] + list(torch.tensor([a for a, _ in seqs]).cumsum(0)), dtype=torch.int32)
