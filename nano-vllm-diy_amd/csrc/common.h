@@ -97,7 +97,6 @@ struct AttnArgs {
   int32_t pf_merge_cap;
   int32_t pf_part_cap;
   int32_t pf_slots;             // persistent work-groups of the prefill kernel
-  int32_t pf_buckets;           // length buckets of the work list (set by the prefill launch)
   int32_t prefill_qtiles;       // upper bound on query tiles per sequence (from max_seqlen_q)
   // Fused decode step (qkv != nullptr): q is the per-head RMSNorm + RoPE of the q part of
   // the fused qkv row of the sequence's token, and the split holding the sequence's last key

@@ -79,7 +79,7 @@ constexpr int kMergeLoads = PK_MERGE_LOADS;  // merge: splits whose outputs load
 // Length buckets of the work list (longest first). prefill_kernel: 4 -> 8 took the dense prompts
 // 144.4 -> 141.6 us and the long chunks 605 -> 594 us, 16 gave 146.3 and 594; prefill_w8_kernel
 // keeps 4 (8: 31 prompts of 512 114.2 -> 118.9 us, 15 chunks of 100 over 4096 keys 117.5 -> 119.9).
-constexpr int kBuckets = PK_PREFILL_BUCKETS;
+constexpr int kLargeBuckets = PK_PREFILL_BUCKETS;
 constexpr int kSmallBuckets = 4;
 constexpr float kLazyLog2 = 8.f;       // reference max moves only when exceeded by 2^8
 
@@ -427,27 +427,30 @@ __device__ __forceinline__ int unit_tiles(const SeqDims& d, int qt) {
 __device__ __forceinline__ int unit_splits(int t, int T) { return t > T ? (t + T - 1) / T : 1; }
 __device__ __forceinline__ int split_begin(int t, int n, int s) { return (int)((unsigned)(t * s) / (unsigned)n); }
 
-// Length bucket of a group of t tiles (0 = longest) of n buckets for split size T.
-__device__ __forceinline__ int length_bucket(int t, int T, int n) {
-  int j = 0;  // the largest j < n with t n > j T (compares, no division)
+// Length bucket of a group of t tiles (0 = longest) of N buckets for split size T.
+template <int N>
+__device__ __forceinline__ int length_bucket(int t, int T) {
+  int j = 0;  // the largest j < N with t N > j T (compares, no division)
 #pragma unroll
-  for (int i = 1; i < kBuckets; ++i) j = i < n && t * n > i * T ? i : j;
-  return n - 1 - j;
+  for (int i = 1; i < N; ++i) j = t * N > i * T ? i : j;
+  return N - 1 - j;
 }
 
 // Work list. Waves take sequences in turn and lanes take a sequence's query tiles, so a
 // long prompt's tiles are planned in parallel. Groups land in their length bucket through
 // LDS cursors: the order inside a bucket depends on timing, but a group's work and the
 // merge order of its splits do not, so results are bit-identical from run to run.
-template <int G, bool CAUSAL>
+template <int G, bool CAUSAL, bool SMALL>
 __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const AttnArgs a) {
   constexpr int TM = kPrefillRows / G;
   constexpr int W = kPlanThreads / kWave;
+  constexpr int kBuckets = SMALL ? kSmallBuckets : kLargeBuckets;
   __shared__ long long red[W];
   __shared__ int cur[kBuckets + 2];  // bucket cursors, partial-group cursor, merge cursor
   // (sequence, Lq, Lk) of the prefill sequences among the first kPlanCache, in any order: the
   // passes read them from LDS and do not walk the decode rows of a mixed batch (128 of them beside
-  // 8 chunks: nine rounds of the wavefronts per pass instead of one, 9.5 us for the plan)
+  // 8 chunks: nine rounds of the wavefronts per pass instead of one, 9.5 us for the plan). SMALL:
+  // all of them, in their own places (the list's barrier and atomics cost a small call 1 us)
   __shared__ int4 dims[kPlanCache];
   __shared__ int listed;
   const int tid = threadIdx.x;
@@ -456,14 +459,19 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const AttnAr
   const int S = a.num_seqs;
   const int hkv = a.num_kv_heads;
 
-  if (tid == 0) listed = 0;
-  __syncthreads();
+  if constexpr (!SMALL) {
+    if (tid == 0) listed = 0;
+    __syncthreads();
+  }
   for (int b = tid; b < min(S, kPlanCache); b += kPlanThreads) {
     const SeqDims d = seq_dims<TM>(a, b);
-    if (d.nq > 0) dims[atomicAdd(&listed, 1)] = make_int4(b, d.Lq, d.Lk, 0);
+    if constexpr (SMALL)
+      dims[b] = make_int4(b, d.Lq, d.Lk, 0);
+    else if (d.nq > 0)
+      dims[atomicAdd(&listed, 1)] = make_int4(b, d.Lq, d.Lk, 0);
   }
   __syncthreads();
-  const int nlist = listed;
+  const int nlist = SMALL ? min(S, kPlanCache) : listed;
   const int nseq = nlist + max(0, S - kPlanCache);  // entries of the passes: the list, then the rest
   auto dims_of = [&](int i, int& b) {
     if (i >= nlist) {
@@ -511,7 +519,7 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const AttnAr
       const int t = unit_tiles<TM, CAUSAL>(d, qt);
       const int n = unit_splits(t, T);
       for (int sp = 0; sp < n; ++sp)
-        atomicAdd(&cur[length_bucket(split_begin(t, n, sp + 1) - split_begin(t, n, sp), T, a.pf_buckets)], 1);
+        atomicAdd(&cur[length_bucket<kBuckets>(split_begin(t, n, sp + 1) - split_begin(t, n, sp), T)], 1);
     }
   }
   __syncthreads();
@@ -538,7 +546,7 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const AttnAr
       for (int sp = 0; sp < n; ++sp) {
         const int tb = split_begin(t, n, sp);
         const int te = split_begin(t, n, sp + 1);
-        const int k = length_bucket(te - tb, T, a.pf_buckets);
+        const int k = length_bucket<kBuckets>(te - tb, T);
         const int grp = start[k] + atomicAdd(&cur[k], 1);
         if (grp < a.pf_item_cap) a.pf_items[grp] = make_int4(b, qt, tb | (te << 16), n > 1 ? pg + sp : -1);
       }
@@ -2112,7 +2120,7 @@ int device_prefill_slots() {
 }
 
 template <int G, bool PAGED, bool CAUSAL>
-hipError_t launch_prefill_gpc(AttnArgs a, hipStream_t stream) {
+hipError_t launch_prefill_gpc(const AttnArgs& a, hipStream_t stream) {
   // Which kernel: the launch bounds' tiles per work-group, if every sequence were as long as they
   // allow (the lengths are on the device). Uniform batches, w8 kernel against prefill_kernel (us
   // per call). Paged: 15 tiles 60.8 / 63.0, 16 74.5 / 81.0, 20 81.4 / 81.5 and 79.6 / 81.5, 31
@@ -2124,12 +2132,13 @@ hipError_t launch_prefill_gpc(AttnArgs a, hipStream_t stream) {
   const int64_t tiles = (int64_t)a.num_seqs * a.prefill_qtiles * ((a.max_seqlen_k + kTileKeys - 1) / kTileKeys) *
                         a.num_kv_heads;
   const bool small = tiles < (int64_t)kSmallTiles * a.pf_slots;
-  a.pf_buckets = small ? kSmallBuckets : kBuckets;
-  hipLaunchKernelGGL((prefill_plan_kernel<G, CAUSAL>), dim3(1), dim3(kPlanThreads), 0, stream, a);
-  if (small)
+  if (small) {
+    hipLaunchKernelGGL((prefill_plan_kernel<G, CAUSAL, true>), dim3(1), dim3(kPlanThreads), 0, stream, a);
     hipLaunchKernelGGL((prefill_w8_kernel<G, PAGED, CAUSAL>), dim3(a.pf_slots), dim3(kPrefillThreads), 0, stream, a);
-  else
+  } else {
+    hipLaunchKernelGGL((prefill_plan_kernel<G, CAUSAL, false>), dim3(1), dim3(kPlanThreads), 0, stream, a);
     hipLaunchKernelGGL((prefill_kernel<G, PAGED, CAUSAL>), dim3(a.pf_slots), dim3(kPfThreads), 0, stream, a);
+  }
   hipLaunchKernelGGL((prefill_merge_kernel<G>), dim3(kMergeGroups), dim3(kMergeThreads), 0, stream, a);
   return hipGetLastError();
 }
