@@ -2126,9 +2126,9 @@ hipError_t launch_prefill_gpc(const AttnArgs& a, hipStream_t stream) {
   // per call). Paged: 15 tiles 60.8 / 63.0, 16 74.5 / 81.0, 20 81.4 / 81.5 and 79.6 / 81.5, 31
   // 115.8 / 118.8, 36 114.9 / 111.7, 37 115.2 / 114.3, 48 124.0 / 119.9, 300 619 / 554. Flat (a
   // prompt's tiles are half the bound): 4 39.7 / 41.1, 8 44.8 / 47.0, 16 103.6 / 104.8, 31 112.9 /
-  // 112.0, 64 108.9 / 104.6, 256 315 / 288. A ragged batch is taken for a larger one: that costs
+  // 112.0, 32 77.4 / 79.4, 64 108.9 / 104.6, 256 315 / 288. A ragged batch is taken for a larger one: that costs
   // at most the few us by which the small calls differ.
-  constexpr int kSmallTiles = PAGED ? 36 : 24;
+  constexpr int kSmallTiles = 36;
   const int64_t tiles = (int64_t)a.num_seqs * a.prefill_qtiles * ((a.max_seqlen_k + kTileKeys - 1) / kTileKeys) *
                         a.num_kv_heads;
   const bool small = tiles < (int64_t)kSmallTiles * a.pf_slots;
