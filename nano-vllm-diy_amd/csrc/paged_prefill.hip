@@ -1411,7 +1411,6 @@ __global__ __launch_bounds__(kPfThreads, 1) void prefill_kernel(const AttnArgs a
   TileCursor<PAGED> cur;
   int koff[kPfLoads], voff[kPfLoads];
   const char *v1, *v2;
-  int vt1, vt2;
   const auto clamp_k = [&]() {
     if (cur.t0 + TN > it.Lk)
       stage_offsets<false>((int)a.k_row_stride, wave, per_item(lane_), it.Lk - 1 - cur.t0, koff);
@@ -1447,13 +1446,11 @@ __global__ __launch_bounds__(kPfThreads, 1) void prefill_kernel(const AttnArgs a
     cur.advance(a, it.b, it.g, btv);
     clamp_k();
     v1 = cur.v;
-    vt1 = cur.t0;
     stage_tile(cur.k, koff, lds0 + kLdsK1 + wrow);
     stage_v(vfirst, tbase, lds0 + kLdsV0 + wrow);
     cur.advance(a, it.b, it.g, btv);
     clamp_k();
     v2 = cur.v;
-    vt2 = cur.t0;
     stage_tile(cur.k, koff, lds0 + kLdsK2 + wrow);
     cur.advance(a, it.b, it.g, btv);
     clamp_k();
@@ -1525,11 +1522,9 @@ __global__ __launch_bounds__(kPfThreads, 1) void prefill_kernel(const AttnArgs a
       int v1s = kLdsV2, v0s = kLdsV0, vns = kLdsV1;                // V tiles n - 1 .. n + 1
       // Body n: loads of K tile n + 3 and V tile n + 1; K tile n + 2 and V tile n land by its end.
       const auto stage = [&](int n) {
-        if (n + 1 < ntiles) stage_v(v1, vt1, lds0 + vns + wrow);
+        if (n + 1 < ntiles) stage_v(v1, tbase + (n + 1) * TN, lds0 + vns + wrow);
         v1 = v2;
-        vt1 = vt2;
         v2 = cur.v;
-        vt2 = cur.t0;
         if (n + 3 < ntiles) stage_tile(cur.k, koff, lds0 + k3s + wrow);
         cur.advance(a, it.b, it.g, btv);
         clamp_k();
@@ -1612,8 +1607,6 @@ bf16x8 k[16];
         lds_barrier();
         rotate();
       }
-      vt2 = cur.t0 - TN;
-      vt1 = vt2 - TN;
       clamp_k();
 #pragma unroll 1
       for (; t0 + TN - 1 <= lim_lo && n < ntiles; ++n, t0 += TN) {

@@ -84,3 +84,57 @@ def test_step_and_tile_edges(gpu, tail, large):
                                    max(a for a, _ in seqs), max(b for _, b in seqs), D ** -0.5, True, None)
     torch.cuda.synchronize()
     assert_close_bf16(out, want, f"tail {tail}")
+
+
+def _paged_nan(seqs, k, v, hkv, bs, width):
+    """Caches and block table of `width` blocks a sequence; every row that holds no key is NaN."""
+    blocks = sum(-(-n // bs) for _, n in seqs)
+    order = torch.randperm(blocks, generator=torch.Generator().manual_seed(1)).tolist()
+    kc, vc = (torch.full((blocks, bs, hkv, D), float("nan"), dtype=torch.bfloat16) for _ in range(2))
+    bt = torch.full((len(seqs), width), -1, dtype=torch.int32)
+    lo = 0
+    for b, (_, n) in enumerate(seqs):
+        for j in range(-(-n // bs)):
+            blk, m = order.pop(), min(bs, n - j * bs)
+            bt[b, j] = blk
+            kc[blk, :m], vc[blk, :m] = k[lo + j * bs:lo + j * bs + m], v[lo + j * bs:lo + j * bs + m]
+        lo += n
+    return kc, vc, bt
+
+
+# key-count bound that takes a call of these tests to the pipelined kernel, whatever its lengths
+BOUND_K = 32768
+
+
+def _check_nan_past_the_end(gpu, seqs, hq, hkv, paged, what):
+    """The rows of K and V that belong to no sequence are NaN (in the cache's blocks, or behind the last
+    flat row, inside one allocation): a row read past a sequence's end makes its tile's outputs NaN."""
+    max_q = max(a for a, _ in seqs)
+    assert len(seqs) * -(-max_q // (256 * hkv // hq)) * (BOUND_K // 64) * hkv >= 36 * 256  # 36 tiles per work-group
+    q, k, v = _batch(seqs, hq, hkv, lambda t, n: 0, 11)
+    cu_q = torch.tensor([0] + list(torch.tensor([a for a, _ in seqs]).cumsum(0)), dtype=torch.int32)
+    cu_k = torch.tensor([0] + list(torch.tensor([b for _, b in seqs]).cumsum(0)), dtype=torch.int32)
+    want = oracle.varlen_attention(q, k, v, cu_q, cu_k, D ** -0.5, True, None)
+    if paged:
+        kd, vd, bt = _paged_nan(seqs, k, v, hkv, 64, BOUND_K // 64)
+    else:
+        pad = torch.full((128, hkv, D), float("nan"), dtype=torch.bfloat16)
+        kd, vd, bt = torch.cat([k, pad]), torch.cat([v, pad]), None
+    kd, vd = kd.to(gpu), vd.to(gpu)
+    if not paged:
+        kd, vd = kd[:len(k)], vd[:len(v)]
+    out = pagedkv.varlen_attention(q.to(gpu), kd, vd, cu_q.to(gpu), cu_k.to(gpu), max_q, BOUND_K,
+                                   D ** -0.5, True, None if bt is None else bt.to(gpu))
+    torch.cuda.synchronize()
+    assert_close_bf16(out, want, what)
+
+
+@pytest.mark.parametrize("paged", [True, False])
+@pytest.mark.parametrize("hq,hkv", [(16, 8), (4, 4), (8, 2), (8, 1)])
+@pytest.mark.parametrize("keys", [63, 65, 127, 129, 191, 193, 255, 257, 319, 321, 383, 449])
+def test_last_tile_of_short_items(gpu, keys, hq, hkv, paged):
+    """Items of 1 to 8 tiles whose last tile ends with the sequence, as the last of a flat batch and,
+    paged, behind a cached prefix too."""
+    print(f"[prefill-range] last tile keys={keys} hq={hq} hkv={hkv} paged={paged}", flush=True)
+    seqs = [(1500, 1500)] + ([(60, keys), (2, keys)] if paged else []) + [(keys, keys)]
+    _check_nan_past_the_end(gpu, seqs, hq, hkv, paged, f"keys={keys} paged={paged}")
