@@ -92,7 +92,8 @@ struct AttnArgs {
                                 // item i = kv head i % Hkv of group i / Hkv
   int4* pf_merges;              // [pf_merge_cap] split units (b, qt, first partial group, splits)
   uint16_t* pf_part_o;          // [part][32 chunks of 4 dims][kPrefillRows][4] the split's output (bf16)
-  float* pf_part_ml;            // [part][kPrefillRows][2] = (running max in the exp2 domain, sum)
+  float* pf_part_ml;            // [part][kPrefillRows][2] = (reference m near the row's max in the exp2 domain,
+                                // sum of 2^(score - m))
   int32_t pf_item_cap;
   int32_t pf_merge_cap;
   int32_t pf_part_cap;

@@ -1714,7 +1714,7 @@ bf16x8 k[16];
         const int tok = done.qt * TM + row % TM;
         if (done.part >= a.pf_part_cap || tok >= done.Lq) continue;
         // The split's own output o / l in bf16 -- as precise as an unsplit row's output -- with
-        // (max, sum) in fp32 for the merge. Chunk-major (chunk = 4 dims = d / 4): one store
+        // (reference, sum) in fp32 for the merge. Chunk-major (chunk = 4 dims = d / 4): one store
         // instruction writes two contiguous 256-byte runs (32 rows x 8 bytes per lane half).
         uint16_t* po = a.pf_part_o + (int64_t)done.part * (32 * kPrefillRows * 4);
 #pragma unroll
@@ -1727,9 +1727,13 @@ bf16x8 k[16];
             w.y = pack_bf16x2(st.o[rb][md][4 * gq + 2] * inv[rb], st.o[rb][md][4 * gq + 3] * inv[rb]);
             *reinterpret_cast<uint2*>(po + ((int64_t)chunk * kPrefillRows + row) * 4) = w;
           }
-        if (half == 0)
+        // The merge takes 2^(reference - largest reference) as a split's scale, so the reference has
+        // to be near the row's max: the sum's exponent, far from 0 here, moves into it.
+        if (half == 0) {
+          const float e = (float)__builtin_amdgcn_frexp_expf(l_tot[rb]);
           *reinterpret_cast<float2*>(a.pf_part_ml + ((int64_t)done.part * kPrefillRows + row) * 2) =
-              make_float2(l_tot[rb] > 0.f ? -st.nm[rb] : -INFINITY, l_tot[rb]);
+              make_float2(l_tot[rb] > 0.f ? e - st.nm[rb] : -INFINITY, __builtin_amdgcn_frexp_mantf(l_tot[rb]));
+        }
       }
     }
     if (next < 0) return;
@@ -1737,7 +1741,8 @@ bf16x8 k[16];
 }
 
 // Merge the partials of every split unit: out = sum_s w_s o_s / sum_s w_s with
-// w_s = exp2(m_s - max_s m_s) l_s, o_s the split's normalised output (bf16). Work item =
+// w_s = exp2(m_s - max_s m_s) l_s, o_s the split's normalised output (bf16), m_s a reference that
+// is near the split's largest score, so that a weight that flushes to 0 is negligible. Work item =
 // (split unit, quarter of head_dim, kv head); thread t owns row t of the unit and 8 chunks
 // of 4 dims. At most 4 wavefronts per SIMD: the register budget lets the loads of
 // kMergeLoads splits be in flight at once. Two rounds of loads reach the first store: the

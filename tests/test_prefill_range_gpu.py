@@ -103,7 +103,7 @@ def _paged_nan(seqs, k, v, hkv, bs, width):
 
 
 # key-count bound that takes a call of these tests to the pipelined kernel, whatever its lengths
-BOUND_K = 32768
+BOUND_K = 1 << 19
 
 
 def _check_nan_past_the_end(gpu, seqs, hq, hkv, paged, what):
@@ -138,3 +138,33 @@ def test_last_tile_of_short_items(gpu, keys, hq, hkv, paged):
     print(f"[prefill-range] last tile keys={keys} hq={hq} hkv={hkv} paged={paged}", flush=True)
     seqs = [(1500, 1500)] + ([(60, keys), (2, keys)] if paged else []) + [(keys, keys)]
     _check_nan_past_the_end(gpu, seqs, hq, hkv, paged, f"keys={keys} paged={paged}")
+
+
+def _check_bound(gpu, q, k, v, seqs, what, causal=True, scale_out=1.0):
+    """The pipelined kernel over a paged copy of k and v, against the oracle (scale_out: a power of two that
+    brings the outputs near 1)."""
+    hkv, max_q = k.shape[1], max(a for a, _ in seqs)
+    assert len(seqs) * -(-max_q // (256 * hkv // q.shape[1])) * (BOUND_K // 64) * hkv >= 36 * 256
+    cu_q = torch.tensor([0] + list(torch.tensor([a for a, _ in seqs]).cumsum(0)), dtype=torch.int32)
+    cu_k = torch.tensor([0] + list(torch.tensor([b for _, b in seqs]).cumsum(0)), dtype=torch.int32)
+    want = oracle.varlen_attention(q, k, v, cu_q, cu_k, D ** -0.5, causal, None)
+    kc, vc, bt = _paged_nan(seqs, k, v, hkv, 64, BOUND_K // 64)
+    out = pagedkv.varlen_attention(q.to(gpu), kc.to(gpu), vc.to(gpu), cu_q.to(gpu), cu_k.to(gpu), max_q, BOUND_K,
+                                   D ** -0.5, causal, bt.to(gpu))
+    torch.cuda.synchronize()
+    assert_close_bf16(out.cpu().float() * scale_out, want.float() * scale_out, what)
+    return out.cpu()
+
+
+@pytest.mark.parametrize("order", ["rise first", "rise last"])
+@pytest.mark.parametrize("steps", [20, 40, 56, 58, 60, 62])
+@pytest.mark.parametrize("hq,hkv", [(16, 8), (4, 4), (8, 1)])
+def test_merge_weighs_splits_by_their_sums(gpu, hq, hkv, steps, order):
+    """Two splits of one unit whose weights differ by 8 to 1 while their references lie far apart: in one
+    the two heavy keys come late (2 log2 per step above its first keys), in the other among the first
+    32, two steps higher."""
+    print(f"[prefill-range] merge hq={hq} hkv={hkv} steps={steps} {order}", flush=True)
+    late, early = (0, 512) if order == "rise first" else (512, 0)
+    heavy = {late + 100: steps, late + 300: steps, early + 8: steps + 2}
+    seqs = [(40, 1024)]     # 16 tiles: two splits of 8
+    _check_bound(gpu, *_batch(seqs, hq, hkv, lambda t, n: heavy.get(t, 0), 5), seqs, f"{steps} {order}")
