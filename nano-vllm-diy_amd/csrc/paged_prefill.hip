@@ -873,7 +873,7 @@ __global__ __launch_bounds__(kPrefillThreads, kWavesPerSimd) void prefill_w8_ker
 // takes 32, up to five independent vector instructions beside it are free, a sixth and further
 // ones cost 4-5, a vector instruction that uses the previous one's result 8, an exponential 8,
 // v_dot2 (which the MFMA pipe executes too) 17, an LDS read beside a full slot 4. Hence: no
-// instruction uses a result of its own slot; sums are additions, not v_dot2; no running max (one
+// instruction uses a result of its own slot; sums by a small MFMA, not v_dot2; no running max (one
 // reference per row and item with 2^124 of room, checked by the sum at the end); K and V bypass
 // the registers. Steady tile 4600 -> 3000 cycles; 16 chunks of 1024 over 4096-token prefixes
 // (618 GFLOP) 647-670 -> 584-617 us per call with the 24 us store (kernel alone 692 -> 591 us in a
@@ -971,7 +971,9 @@ struct PfState {
   u32x4 p[2][kPfRB][2];        // P (bf16 pairs) of steps of either parity
   bf16x8 kf[kPfAhead];         // K operands read ahead
   float nm[kPfRB];             // minus the reference max of the exponentials
-  float l[kPfRB];              // row sums over this lane's keys
+  u32x2 ones;                  // four 1.0 in bf16
+  f32x4 ls[kPfRB];             // the tile loops' row sums over this lane's keys (four equal values)
+  float l[kPfRB];              // the item's
 };
 
 __device__ __forceinline__ bf16x8 read_k(const lds_char* sK, const TileLanes& tl, int kb) {
@@ -1010,6 +1012,17 @@ __device__ __forceinline__ void mfma_o(f32x16& o, const bf16x8& v, const u32x4& 
   asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(o) : "v"(v), "v"(p));
 }
 
+// Row sums += the four keys of p (ones times P^T, 4 x 4 x 4 in 16 blocks: a lane's result is the sum of
+// its own four). The sums take the rounded P of the P.V product, so that numerator and denominator
+// weigh every key alike: a key far above the others gives its V row exactly, where a sum of the
+// unrounded p is off by up to 2^-9. Issued right before a slot's large MFMA it costs the 8 cycles that it
+// runs and saves the additions: 16 chunks of 1024 over 4096-token prefixes 584 (unrounded sums) -> 591
+// us; after the large MFMA, where it holds up the vector instructions, 600; unpacking the rounded
+// pairs for vector additions 609.
+__device__ __forceinline__ void mfma_sum(f32x4& l, const u32x2& ones, const u32x2& p) {
+  asm volatile("v_mfma_f32_4x4x4_16b_bf16 %0, %1, %2, %0" : "+a"(l) : "a"(ones), "v"(p));
+}
+
 // The first softmax of an item (step 0): the reference is the row's max over the step's keys
 // raised by kHeadroomLog2, P = 2^(s - reference) in bf16. Later steps keep the reference.
 __device__ __forceinline__ void softmax_first(PfState& st, int t0, const int (&lim)[kPfRB], float scale_log2,
@@ -1025,17 +1038,14 @@ __device__ __forceinline__ void softmax_first(PfState& st, int t0, const int (&l
     for (int rr = 1; rr < 16; ++rr) t = fmaxf(t, s[rr]);
     t = swap_halves_max(t) * scale_log2;
     const float nm = t == -INFINITY ? 0.f : -t - kHeadroomLog2;
-    float ps = 0.f;
 #pragma unroll
     for (int i = 0; i < 16; i += 2) {
       const float p0 = exp2_fast(__builtin_fmaf(s[i], scale_log2, nm));
       const float p1 = exp2_fast(__builtin_fmaf(s[i + 1], scale_log2, nm));
       const bf16x2 pr = {static_cast<__bf16>(p0), static_cast<__bf16>(p1)};
       st.p[0][rb][i >> 3][(i & 7) >> 1] = __builtin_bit_cast(uint32_t, pr);
-      ps += p0 + p1;
     }
     st.nm[rb] = nm;
-    st.l[rb] = ps;
   }
 }
 
@@ -1053,12 +1063,7 @@ __device__ __forceinline__ void pf_iteration(PfState& st, const lds_char* sK, co
   constexpr int KB = kHeadDim / 16;
   constexpr int NE = 16 * kPfRB;  // scores per lane
   bf16x8 kf[KB], vf[8];
-  float ps[kPfRB];
   float x[NE];  // a score on its way to p
-#pragma unroll
-  for (int rb = 0; rb < kPfRB; ++rb) {
-    ps[rb] = 0.f;
-  }
 #pragma unroll
   for (int j = 0; j < kPfAhead; ++j) kf[j] = st.kf[j];
   // elements started by the end of slot s: 32 of them in 29 slots, so the last is packed in slot 31
@@ -1081,17 +1086,19 @@ __device__ __forceinline__ void pf_iteration(PfState& st, const lds_char* sK, co
     }
     // MFMAs
     if (sl < 16) {
+      if (sl & 1) {  // the sum of step i - 1, row block 1's last keys (packed in slot 31) at the end
+        const u32x4 p = st.p[NXT][sl >> 3][(sl >> 2) & 1];
+        mfma_sum(st.ls[sl >> 3], st.ones, (sl & 2) ? u32x2{p[2], p[3]} : u32x2{p[0], p[1]});
+      }
       mfma_s(st.s[NXT][sl & 1], kf[sl / 2], st.q[sl & 1][sl / 2], sl < 2, sl & 1);
     } else {
       const int fv = (sl - 16) / 2, rb = sl & 1;
       mfma_o(st.o[rb][fv & 3], vf[fv], st.p[NXT][rb][fv >> 2]);
     }
     // softmax: the scale and reference of some elements, the exponentials of those of the slot
-    // before, sum and packing of those of the slot before that
+    // before, packing of those of the slot before that
 #pragma unroll
     for (int e = nf(sl - 4); e < nf(sl - 3); ++e) {
-      ps[e >> 4] += x[e];
-      asm volatile("" ::"v"(ps[e >> 4]));  // here, not after the loop
       if (e & 1) {
         const bf16x2 pr = {static_cast<__bf16>(x[e - 1]), static_cast<__bf16>(x[e])};
         st.p[CUR][e >> 4][(e & 15) >> 3][(e & 7) >> 1] = __builtin_bit_cast(uint32_t, pr);
@@ -1112,7 +1119,6 @@ __device__ __forceinline__ void pf_iteration(PfState& st, const lds_char* sK, co
   }
 #pragma unroll
   for (int rb = 0; rb < kPfRB; ++rb) {
-    st.l[rb] += ps[rb];
     // S is final here (the MFMAs that wrote it are 16 MFMAs back), and P is computed before here
     asm volatile("" : "+v"(st.s[NXT][rb]), "+v"(st.p[CUR][rb][0]), "+v"(st.p[CUR][rb][1]));
   }
@@ -1473,11 +1479,14 @@ __global__ __launch_bounds__(kPfThreads, 1) void prefill_kernel(const AttnArgs a
       lim_lo = min(lim_lo, CAUSAL ? min(it.Lk - 1, blo + P) : it.Lk - 1);
       lim_hi = max(lim_hi, CAUSAL ? min(it.Lk - 1, blo + 31 + P) : it.Lk - 1);
       st.nm[rb] = 0.f;
-      st.l[rb] = 0.f;
     }
     const auto clear_o = [&]() {
+      st.ones = u32x2{0x3f803f80u, 0x3f803f80u};
+      asm volatile("" : "+a"(st.ones));
 #pragma unroll
-      for (int rb = 0; rb < kPfRB; ++rb)
+      for (int rb = 0; rb < kPfRB; ++rb) {
+        st.ls[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        asm volatile("" : "+a"(st.ls[rb]));
 #pragma unroll
         for (int md = 0; md < 4; ++md) {
           const float zero = __int_as_float(per_item(0));
@@ -1485,6 +1494,7 @@ __global__ __launch_bounds__(kPfThreads, 1) void prefill_kernel(const AttnArgs a
           for (int rr = 0; rr < 16; ++rr) st.o[rb][md][rr] = zero;
           asm volatile("" : "+a"(st.o[rb][md]));
         }
+      }
     };
     // steps (32 keys) this wavefront's rows see
     const int nw = min(2 * ntiles, (lim_hi - tbase + kStepKeys) >> 5);
@@ -1591,7 +1601,7 @@ bf16x8 k[16];
       // would count the loop's own loads)
 #pragma unroll
       for (int rb = 0; rb < kPfRB; ++rb)
-        asm volatile("" : "+v"(st.s[1][rb]), "+v"(st.p[0][rb][0]), "+v"(st.p[0][rb][1]), "+v"(st.nm[rb]), "+v"(st.l[rb]));
+        asm volatile("" : "+v"(st.s[1][rb]), "+v"(st.p[0][rb][0]), "+v"(st.p[0][rb][1]), "+v"(st.nm[rb]));
 #pragma unroll 1
       for (; t0 + TN - 1 <= lim_lo && n + 4 < ntiles; ++n, t0 += TN) {
         const lds_char* const ks = smem + k0s;
@@ -1638,6 +1648,8 @@ bf16x8 k[16];
     bool bad = false;
 #pragma unroll
     for (int rb = 0; rb < kPfRB; ++rb) {
+      asm volatile("" : "+a"(st.ls[rb]));
+      st.l[rb] = st.ls[rb][0];
       l_tot[rb] = swap_halves_sum(st.l[rb]);
       bad |= !(l_tot[rb] <= kSumLimit) || (l_tot[rb] == 0.f && lim[rb] >= tbase);
     }

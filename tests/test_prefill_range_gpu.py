@@ -168,3 +168,17 @@ def test_merge_weighs_splits_by_their_sums(gpu, hq, hkv, steps, order):
     heavy = {late + 100: steps, late + 300: steps, early + 8: steps + 2}
     seqs = [(40, 1024)]     # 16 tiles: two splits of 8
     _check_bound(gpu, *_batch(seqs, hq, hkv, lambda t, n: heavy.get(t, 0), 5), seqs, f"{steps} {order}")
+
+
+@pytest.mark.parametrize("hq,hkv", [(16, 8), (4, 4), (8, 1)])
+@pytest.mark.parametrize("key", [5, 40, 130, 500])
+def test_one_heavy_key_gives_its_value_exactly(gpu, hq, hkv, key):
+    """A key 40 log2 above all others: numerator and denominator weigh it by the same rounded p, so every row
+    is its V row, bit for bit, whatever the fraction that p was rounded from."""
+    print(f"[prefill-range] heavy key={key} hq={hq} hkv={hkv}", flush=True)
+    seqs = [(100, 560), (300, 560)]
+    q, k, v = _batch(seqs, hq, hkv, lambda t, n: 20 if t == key else 0, 3 + key)
+    out = _check_bound(gpu, q, k, v, seqs, f"key {key}")
+    seen = torch.cat([torch.arange(a) + b - a >= key for a, b in seqs])
+    rows = torch.cat([torch.full((a,), i) for i, (a, _) in enumerate(seqs)]) * 560 + key
+    assert torch.equal(out[seen], v[rows][seen].repeat_interleave(hq // hkv, 1))
