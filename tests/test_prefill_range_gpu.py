@@ -182,3 +182,16 @@ def test_one_heavy_key_gives_its_value_exactly(gpu, hq, hkv, key):
     seen = torch.cat([torch.arange(a) + b - a >= key for a, b in seqs])
     rows = torch.cat([torch.full((a,), i) for i, (a, _) in enumerate(seqs)]) * 560 + key
     assert torch.equal(out[seen], v[rows][seen].repeat_interleave(hq // hkv, 1))
+
+
+@pytest.mark.parametrize("steps", [0, 30, 55])
+@pytest.mark.parametrize("exponent", [-100, -70, 70, 110])
+@pytest.mark.parametrize("hq,hkv", [(16, 8), (4, 4), (8, 1)])
+def test_values_of_any_magnitude(gpu, hq, hkv, exponent, steps):
+    """V rows far from 1 beside scores that rise by up to 112 log2 over an item: neither the products p v nor
+    their sums may leave the range of fp32 where the output does not."""
+    print(f"[prefill-range] V 2^{exponent} steps={steps} hq={hq} hkv={hkv}", flush=True)
+    seqs = [(130, 700), (300, 333)]
+    q, k, v = _batch(seqs, hq, hkv, lambda t, n: steps if t % 90 == 77 else 0, 9)
+    v = (v.float() * 2.0 ** exponent).to(torch.bfloat16)
+    _check_bound(gpu, q, k, v, seqs, f"V 2^{exponent}, steps {steps}", scale_out=2.0 ** -exponent)
