@@ -1642,9 +1642,10 @@ bf16x8 k[16];
       }
     }
     // The sum shows whether the item's reference held: a row whose scores rose beyond the limit (or
-    // that overflowed on the way), or whose sum vanished, has the whole item done again with a running
-    // max. So has one whose O is not finite where the sum is above what a running max could have left
-    // (p up to 2^kLazyLog2 for every key): large V rows overflow there beside sums within the limit.
+    // that overflowed on the way), or that never reached its reference (first keys of -infinity leave
+    // it at 0, wherever the others lie), has the whole item done again with a running max. So has one
+    // whose O is not finite where the sum is above what a running max could have left (p up to
+    // 2^kLazyLog2 for every key): large V rows overflow there beside sums within the limit.
     float l_tot[kPfRB];
     bool bad = false, large = false;
 #pragma unroll
@@ -1652,7 +1653,7 @@ bf16x8 k[16];
       asm volatile("" : "+a"(st.ls[rb]));
       st.l[rb] = st.ls[rb][0];
       l_tot[rb] = swap_halves_sum(st.l[rb]);
-      bad |= !(l_tot[rb] <= kSumLimit) || (l_tot[rb] == 0.f && lim[rb] >= tbase);
+      bad |= !(l_tot[rb] <= kSumLimit) || (l_tot[rb] < 0.5f && lim[rb] >= tbase);
       large |= l_tot[rb] > (float)(TN << (int)kLazyLog2) * (float)ntiles;
     }
     if (__builtin_amdgcn_ballot_w64(large) != 0) {

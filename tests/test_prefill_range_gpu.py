@@ -195,3 +195,14 @@ def test_values_of_any_magnitude(gpu, hq, hkv, exponent, steps):
     q, k, v = _batch(seqs, hq, hkv, lambda t, n: steps if t % 90 == 77 else 0, 9)
     v = (v.float() * 2.0 ** exponent).to(torch.bfloat16)
     _check_bound(gpu, q, k, v, seqs, f"V 2^{exponent}, steps {steps}", scale_out=2.0 ** -exponent)
+
+
+@pytest.mark.parametrize("hq,hkv", [(16, 8), (4, 4), (8, 1)])
+def test_first_keys_of_minus_infinity(gpu, hq, hkv):
+    """The first 32 keys score -infinity (bf16's lowest value in K), the others so low that without a reference
+    of their own 2^score is below fp32's normal range for most of them."""
+    print(f"[prefill-range] -inf first hq={hq} hkv={hkv}", flush=True)
+    seqs = [(260, 300)]     # every row sees more than 32 keys
+    q, k, v = _batch(seqs, hq, hkv, lambda t, n: -61 if t == 35 else -62, 4)
+    k[:32, :, 0] = torch.finfo(torch.bfloat16).min
+    _check_bound(gpu, q, k, v, seqs, "-inf first")
