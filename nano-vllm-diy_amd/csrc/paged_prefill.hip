@@ -1223,17 +1223,21 @@ __device__ __forceinline__ int per_item(int v) {
 
 // An item's tiles one after the other with a running row max (numerator and sum rescaled when it
 // moves by more than 2^kLazyLog2): what an item takes whose scores leave the range that one
-// reference covers. Ends with a barrier.
-template <int G, bool PAGED>
+// reference covers. A row block leaves out the steps that none of its rows sees (their p is 0, but a V
+// row of infinities or NaN would reach O as 0 * infinity). Ends with a barrier.
+template <int G, bool PAGED, bool CAUSAL>
 __device__ __forceinline__ void prefill_item_safe(const AttnArgs& a, PfState& st, const PfItem& it, int bt_lane,
                                                   const int (&lim)[kPfRB], lds_char* const smem, int wave, int lane) {
   constexpr int TM = kPrefillRows / G;
   const int b = it.b, g = it.g, k0 = it.k0, Lk = it.Lk, tbase = it.tb * kTileKeys, ntiles = it.te - it.tb;
   const int half = lane >> 5;
+  int lim_hi[kPfRB];  // the last key that a row of the block sees
   // Q again (the tile loops' operands need not outlive them)
 #pragma unroll
   for (int rb = 0; rb < kPfRB; ++rb) {
     const int row = block_row<G>(wave, rb) + (lane & 31);
+    const int blo = it.qt * TM + block_row<G>(wave, rb) % TM;
+    lim_hi[rb] = CAUSAL ? min(Lk - 1, blo + 31 + Lk - it.Lq) : Lk - 1;
     const int tok = min(it.qt * TM + row % TM, it.Lq - 1);
     const uint16_t* qp = a.q + (int64_t)(it.q0 + tok) * a.q_row_stride + (g * G + row / TM) * kHeadDim + 8 * half;
 #pragma unroll
@@ -1272,6 +1276,7 @@ __device__ __forceinline__ void prefill_item_safe(const AttnArgs& a, PfState& st
       const lds_char* const sV = smem + kTileBytes + hs * 32 * kRowBytes;
 #pragma unroll
       for (int rb = 0; rb < kPfRB; ++rb) {
+        if (t0 + hs * kStepKeys > lim_hi[rb]) continue;
         f32x16 s[1];
 #pragma unroll
         for (int rr = 0; rr < 16; ++rr) s[0][rr] = 0.f;
@@ -1470,6 +1475,7 @@ __global__ __launch_bounds__(kPfThreads, 1) void prefill_kernel(const AttnArgs a
     const int P = it.Lk - it.Lq;
     int lim[kPfRB];
     int lim_lo = 0x7fffffff, lim_hi = -1;  // keys <= lim_lo: seen by all the wavefront's rows, > lim_hi: by none
+    int lim_hi0 = -1;                      // > lim_hi0: by none of the first block's
 #pragma unroll
     for (int rb = 0; rb < kPfRB; ++rb) {
       const int r0 = block_row<G>(wave, rb);  // 32 tokens of one head
@@ -1478,6 +1484,7 @@ __global__ __launch_bounds__(kPfThreads, 1) void prefill_kernel(const AttnArgs a
       lim[rb] = min(it.te * TN, CAUSAL ? min(it.Lk, blo + col + P + 1) : it.Lk) - 1;
       lim_lo = min(lim_lo, CAUSAL ? min(it.Lk - 1, blo + P) : it.Lk - 1);
       lim_hi = max(lim_hi, CAUSAL ? min(it.Lk - 1, blo + 31 + P) : it.Lk - 1);
+      if (rb == 0) lim_hi0 = lim_hi;
       st.nm[rb] = 0.f;
     }
     const auto clear_o = [&]() {
@@ -1656,6 +1663,9 @@ bf16x8 k[16];
       bad |= !(l_tot[rb] <= kSumLimit) || (l_tot[rb] < 0.5f && lim[rb] >= tbase);
       large |= l_tot[rb] > (float)(TN << (int)kLazyLog2) * (float)ntiles;
     }
+    // With one head per unit a wavefront's second block may see a tile that its first does not, whose V
+    // rows reach the first's O as 0 * V: the same look for what is not finite.
+    if constexpr (G == 1) large |= ntiles > 0 && tbase + (nw - 1) / 2 * TN > lim_hi0;
     if (__builtin_amdgcn_ballot_w64(large) != 0) {
       float z = 0.f;  // NaN if any is not finite
 #pragma unroll
@@ -1671,7 +1681,7 @@ bf16x8 k[16];
     if (ntiles > 0 && __builtin_amdgcn_ballot_w64(bad) != 0 && lane == 0) *redo = 1;
     lds_barrier();  // every wavefront is done with the item's tiles
     if (__builtin_expect(ntiles > 0 && __builtin_amdgcn_readfirstlane(*redo) != 0, 0)) {
-      prefill_item_safe<G, PAGED>(a, st, it, btv, lim, smem, wave, per_item(lane_));
+      prefill_item_safe<G, PAGED, CAUSAL>(a, st, it, btv, lim, smem, wave, per_item(lane_));
 #pragma unroll
       for (int rb = 0; rb < kPfRB; ++rb) l_tot[rb] = swap_halves_sum(st.l[rb]);
     }

@@ -206,3 +206,32 @@ def test_first_keys_of_minus_infinity(gpu, hq, hkv):
     q, k, v = _batch(seqs, hq, hkv, lambda t, n: -61 if t == 35 else -62, 4)
     k[:32, :, 0] = torch.finfo(torch.bfloat16).min
     _check_bound(gpu, q, k, v, seqs, "-inf first")
+
+
+@pytest.mark.parametrize("steps", ["flat", "jump", "ramp"])
+@pytest.mark.parametrize("prefix", [0, 16, 48])
+@pytest.mark.parametrize("hq,hkv", [(16, 8), (4, 4), (8, 1)])
+def test_non_finite_values_stay_behind_the_causal_limit(gpu, hq, hkv, prefix, steps):
+    """NaN and infinities in a V row reach rows whose block of 32 ends in an earlier 64-key tile in no way, also
+    where the scores need a running maximum."""
+    print(f"[prefill-range] non-finite V hq={hq} hkv={hkv} prefix={prefix} {steps}", flush=True)
+    lq, bad = 700, 330
+    seqs = [(lq, lq + prefix)]
+    fn = STEPS[steps] if steps != "flat" else lambda t, n: 0
+    q, k, v = _batch(seqs, hq, hkv, fn, 8)
+    assert -(-lq // (256 * hkv // hq)) * (BOUND_K // 64) * hkv >= 36 * 256
+    hot = v.clone()
+    hot[bad, :, ::2] = float("nan")
+    hot[bad, :, 1::2] = float("inf")
+    cu_q = torch.tensor([0, lq], dtype=torch.int32)
+    cu_k = torch.tensor([0, lq + prefix], dtype=torch.int32)
+    want = oracle.varlen_attention(q, k, v, cu_q, cu_k, D ** -0.5, True, None)
+    kc, vc, bt = _paged_nan(seqs, k, hot, hkv, 64, BOUND_K // 64)
+    out = pagedkv.varlen_attention(q.to(gpu), kc.to(gpu), vc.to(gpu), cu_q.to(gpu), cu_k.to(gpu), lq, BOUND_K,
+                                   D ** -0.5, True, bt.to(gpu))
+    torch.cuda.synchronize()
+    last = torch.arange(lq) // 32 * 32 + 31 + prefix      # the last key that a row's block of 32 sees
+    clean = last < bad // 64 * 64
+    assert clean.sum() > 200
+    assert_close_bf16(out.cpu()[clean], want[clean], "rows before the non-finite key")
+    assert not out.cpu()[bad + 64 - prefix:].isfinite().any()
