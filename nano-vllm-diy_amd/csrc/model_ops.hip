@@ -10,6 +10,8 @@
 // the reference (F.linear on bf16 operands); the greedy choice here compares the fp32 dot
 // products after rounding them to bf16 and keeps the lowest vocabulary index among equal
 // maxima, which is what argmax over the bf16 logits returns.
+#include <algorithm>
+
 #include "common.h"
 
 namespace pk {
@@ -237,22 +239,155 @@ __global__ __launch_bounds__(kLmThreads, 2) void lm_head_greedy_kernel(
   }
 }
 
-// Variant for hidden <= kLmSplitMaxK: a persistent work-group per CU walks 32-row vocabulary tiles,
-// and its eight wavefronts split K: wavefront w multiplies columns [128 w, 128 w + 128) of the
-// tile by those of up to 128 hidden rows, which it holds in registers for the whole call (32 RT of
-// them). A wavefront's slice of a tile (32 rows x 256 bytes) goes from memory to its own 8 KiB of
-// LDS without registers, four full rows' pieces per instruction, one tile ahead and without a
-// barrier; the eight partial sums of a tile meet in the same LDS, two row blocks at a time.
+// Resident variant for hidden <= kLmResidentMaxK: a persistent work-group (one per CU) keeps
+// its group of up to 64 hidden rows in LDS for the whole call and walks vocabulary tiles,
+// so the hidden rows cross from L2 once per work-group instead of once per tile. The
+// `groups` work-groups that cover the row groups of one vocabulary sequence have linear
+// ids l, l + 8, ... and so sit on one XCD: each weight tile comes from HBM once and is
+// shared through that XCD's L2.
+constexpr int kLmResidentMaxK = 1024;
+constexpr int kLmResidentRows = 64;
+constexpr int kLmResidentWaves = 8;
+constexpr int kLmResidentThreads = kLmResidentWaves * 64;
+constexpr int kLmResidentTile = kLmResidentWaves * 32;  // vocabulary rows per tile
+
+template <int RT>
+__global__ __launch_bounds__(kLmResidentThreads, 1) void lm_head_resident_kernel(
+    const uint16_t* __restrict__ x, int64_t x_stride, const int32_t* __restrict__ cu_rows,
+    const uint16_t* __restrict__ w, int64_t w_stride, int32_t rows, int32_t vocab, int32_t k_dim,
+    int32_t groups, unsigned long long* __restrict__ keys) {
+  constexpr int MT = 32 * RT;
+  constexpr int kRowElems = kLmResidentMaxK + 8;  // staged row with a 16-byte pad
+  __shared__ __attribute__((aligned(16))) uint16_t xs[MT * kRowElems];
+  __shared__ unsigned long long best_s[kLmResidentWaves][MT];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = threadIdx.x / kWave;
+  const int r = lane & 31, h = lane >> 5;
+  const int j = blockIdx.x >> 3;
+  const int rg = j % groups;                          // row group
+  const int rank = (j / groups) * 8 + (blockIdx.x & 7);  // position in the vocabulary walk
+  const int nrank = gridDim.x / groups;
+  const int m0 = rg * MT;
+
+  // stage the group's hidden rows (the last row of sequence m when selecting,
+  // llm_head.py:61-63; padded sequences and rows past `rows` stage zeros)
+  const int pieces = k_dim / 8;
+  for (int p = threadIdx.x; p < MT * pieces; p += kLmResidentThreads) {
+    const int row = p / pieces, piece = p - row * pieces;
+    const int m = m0 + row;
+    uint4 val = make_uint4(0, 0, 0, 0);
+    if (m < rows) {
+      const int src = cu_rows != nullptr ? cu_rows[m + 1] - 1 : m;
+      if (src >= 0) val = *reinterpret_cast<const uint4*>(x + (int64_t)src * x_stride + piece * 8);
+    }
+    *reinterpret_cast<uint4*>(xs + row * kRowElems + piece * 8) = val;
+  }
+  __syncthreads();
+
+  unsigned long long best[RT];
+#pragma unroll
+  for (int t = 0; t < RT; ++t) best[t] = 0;
+  // One stream of (tile, chunk) steps: the weight chunk of step n + 2 is in flight while
+  // step n runs, across tile boundaries too.
+  const int ntiles = (vocab + kLmResidentTile - 1) / kLmResidentTile;
+  const int nchunks = k_dim / kLmKChunk;
+  const int my_tiles = rank < ntiles ? (ntiles - rank + nrank - 1) / nrank : 0;
+  const int steps = my_tiles * nchunks;
+  auto wchunk = [&](int step) {
+    const int t = step / nchunks;
+    const int c = step - t * nchunks;
+    const int v_row = (rank + t * nrank) * kLmResidentTile + wave * 32 + r;
+    return w + (int64_t)(v_row < vocab ? v_row : vocab - 1) * w_stride + 64 * h + c * kLmKChunk;
+  };
+  f32x16 acc[RT];
+  auto run_step = [&](const uint4 (&a)[8], int step) {
+    const int t = step / nchunks;
+    const int c = step - t * nchunks;
+    if (c == 0) {
+#pragma unroll
+      for (int q = 0; q < RT; ++q)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[q][i] = 0.f;
+    }
+#pragma unroll
+    for (int s8 = 0; s8 < 8; ++s8) {
+      const bf16x8_t av = __builtin_bit_cast(bf16x8_t, a[s8]);
+#pragma unroll
+      for (int q = 0; q < RT; ++q) {
+        const uint4 bw = *reinterpret_cast<const uint4*>(xs + (32 * q + r) * kRowElems + c * kLmKChunk + 64 * h + 8 * s8);
+        acc[q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, __builtin_bit_cast(bf16x8_t, bw), acc[q], 0, 0, 0);
+      }
+    }
+    if (c == nchunks - 1) {
+      // D layout: lane holds column (hidden row) 32 q + r and vocab rows 8 (i >> 2) + 4 h + (i & 3)
+      const int v_base = (rank + t * nrank) * kLmResidentTile + wave * 32;
+#pragma unroll
+      for (int q = 0; q < RT; ++q)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int v = v_base + 8 * (i >> 2) + 4 * h + (i & 3);
+          if (v < vocab) {
+            const unsigned long long key = logit_key(round_to_bf16(acc[q][i]), (uint32_t)v);
+            best[q] = key > best[q] ? key : best[q];
+          }
+        }
+    }
+  };
+  uint4 a0[8], a1[8];
+  if (steps > 0) {
+    const uint16_t* p0 = wchunk(0);
+#pragma unroll
+    for (int s8 = 0; s8 < 8; ++s8) a0[s8] = *reinterpret_cast<const uint4*>(p0 + 8 * s8);
+  }
+  if (steps > 1) {
+    const uint16_t* p1 = wchunk(1);
+#pragma unroll
+    for (int s8 = 0; s8 < 8; ++s8) a1[s8] = *reinterpret_cast<const uint4*>(p1 + 8 * s8);
+  }
+  for (int step = 0; step < steps; step += 2) {
+    run_step(a0, step);
+    if (step + 2 < steps) {
+      const uint16_t* pn = wchunk(step + 2);
+#pragma unroll
+      for (int s8 = 0; s8 < 8; ++s8) a0[s8] = *reinterpret_cast<const uint4*>(pn + 8 * s8);
+    }
+    if (step + 1 >= steps) break;
+    run_step(a1, step + 1);
+    if (step + 3 < steps) {
+      const uint16_t* pn = wchunk(step + 3);
+#pragma unroll
+      for (int s8 = 0; s8 < 8; ++s8) a1[s8] = *reinterpret_cast<const uint4*>(pn + 8 * s8);
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < RT; ++t) {
+    const unsigned long long other = __shfl_xor(best[t], 32, kWave);
+    const unsigned long long b = other > best[t] ? other : best[t];
+    if (h == 0) best_s[wave][32 * t + r] = b;
+  }
+  __syncthreads();
+  for (int q = threadIdx.x; q < MT; q += kLmResidentThreads) {
+    unsigned long long b = best_s[0][q];
+#pragma unroll
+    for (int wv = 1; wv < kLmResidentWaves; ++wv) b = best_s[wv][q] > b ? best_s[wv][q] : b;
+    if (m0 + q < rows) atomicMax(keys + m0 + q, b);
+  }
+}
+
+// Variant for up to 64 hidden rows of kLmSplitHidden columns: a persistent work-group per CU walks
+// 32-row vocabulary tiles, and its eight wavefronts split K: wavefront w multiplies columns
+// [128 w, 128 w + 128) of the tile by those of the hidden rows, which it holds in registers for the
+// whole call (32 RT of them). A wavefront's slice of a tile (32 rows x 256 bytes) goes from memory to
+// its own 8 KiB of LDS without registers, four full rows' pieces per instruction, one tile ahead and
+// without a barrier; the eight partial sums of a tile meet in the same LDS.
 //
-// What bounded the version before (64 hidden rows in LDS, every lane loading its vocabulary row
-// in 16-byte pieces): each load instruction touched 64 cache lines, 16 bytes of each, so the L1's
-// tag rate bounded it, and 65..128 hidden rows read every weight twice through L2. 97 rows
-// 91.5 us, 3.4 TB/s. Now (us, before -> after, whole call): 1 row 61.4 -> 56.1, 16 62.5 -> 56.8,
-// 64 68.6 -> 67.0, 80 91.1 -> 81.0, 97 91.5 -> 89.1, 128 94.3 -> 89.9. What is left: without the
-// sums over the slices 97 rows take 69 us, without the weight loads 80: the wavefronts' MFMAs
-// and sums alternate behind barriers.
-constexpr int kLmSplitMaxK = 1024;
+// What bounds lm_head_resident_kernel: every lane loads its own vocabulary row, so each load
+// instruction touches 64 cache lines, 16 bytes of each, at the L1's tag rate. Whole call over 151936
+// vocabulary rows, us, that kernel -> this one: 1 row 62.0 -> 54.5, 32 64.3 -> 61.5, 64 68.7 -> 63.8.
+// What is left: the wavefronts' MFMAs and sums alternate behind barriers. Which calls take it:
+// lm_split_pays.
 constexpr int kLmSplitWaves = 8;
+constexpr int kLmSplitHidden = kLmSplitWaves * kLmKChunk;  // 1024: every wavefront has a K slice
 constexpr int kLmSplitThreads = kLmSplitWaves * 64;
 constexpr int kLmSplitRows = 128;       // hidden rows per work-group
 constexpr int kLmSplitTile = 32;        // vocabulary rows per tile
@@ -289,23 +424,16 @@ __device__ __forceinline__ void lm_barrier() {
 template <int RT>
 __global__ __launch_bounds__(kLmSplitThreads, 2) void lm_head_split_kernel(
     const uint16_t* __restrict__ x, int64_t x_stride, const int32_t* __restrict__ cu_rows,
-    const uint16_t* __restrict__ w, int64_t w_stride, int32_t rows, int32_t vocab, int32_t k_dim,
-    int32_t groups, unsigned long long* __restrict__ keys) {
-  constexpr int kRounds = (RT + 1) / 2;  // two row blocks of partial sums fill a slice
+    const uint16_t* __restrict__ w, int64_t w_stride, int32_t rows, int32_t vocab,
+    unsigned long long* __restrict__ keys) {
+  static_assert(RT <= 2, "two row blocks of partial sums fill a slice");
   __shared__ __attribute__((aligned(1024))) char smem_[2 * kLmStageBytes];
   lds_char* const smem = (lds_char*)smem_;
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int r = lane & 31, h = lane >> 5;
-  // the `groups` work-groups of one place in the vocabulary walk (row groups of 128) have linear
-  // ids l, l + 8, ... and so share an XCD's L2
-  const int j = blockIdx.x >> 3;
-  const int rg = j % groups;
-  const int rank = (j / groups) * 8 + (blockIdx.x & 7);
-  const int nrank = gridDim.x / groups;
-  const int m0 = rg * kLmSplitRows;
-  const int nw = k_dim / kLmKChunk;       // wavefronts with a K slice
-  const bool on = wave < nw;
+  const int rank = blockIdx.x;
+  const int nrank = gridDim.x;
   const int slice0 = (int)(uintptr_t)smem + wave * kLmSliceBytes;  // this wavefront's slice, stage 0
   lds_char* const own = smem + wave * kLmSliceBytes;
   // load i of a slice: rows 4 i + (lane >> 4), 16-byte chunk c of row n in slot c ^ (n & 15)
@@ -325,7 +453,7 @@ __global__ __launch_bounds__(kLmSplitThreads, 2) void lm_head_split_kernel(
   const auto load_x = [&](int q) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const int src = src_row(m0 + 32 * q + 4 * i + lrow);
+      const int src = src_row(32 * q + 4 * i + lrow);
       if (src >= 0) {
         const uint16_t* p = x + (int64_t)src * x_stride + wave * kLmKChunk + (lchunk ^ (4 * (i & 3))) * 8;
         asm volatile(
@@ -333,35 +461,32 @@ __global__ __launch_bounds__(kLmSplitThreads, 2) void lm_head_split_kernel(
             "s_nop 0\n\t"
             "global_load_lds_dwordx4 %1, off"
             :
-            : "s"(__builtin_amdgcn_readfirstlane(slice0 + (q & 1) * kLmStageBytes + 1024 * i)), "v"(p)
+            : "s"(__builtin_amdgcn_readfirstlane(slice0 + q * kLmStageBytes + 1024 * i)), "v"(p)
             : "m0", "memory");
       }
     }
   };
   const auto take_x = [&](int q) {
-    const bool live = src_row(m0 + 32 * q + r) >= 0;
+    const bool live = src_row(32 * q + r) >= 0;
 #pragma unroll
     for (int s8 = 0; s8 < 8; ++s8) {
-      const u32x4_t v = read(q & 1, s8);
+      const u32x4_t v = read(q, s8);
       xr[q][s8] = live ? v : u32x4_t{0, 0, 0, 0};
     }
   };
-  if (on) {
-    load_x(0);
-    if constexpr (RT > 1) load_x(1);
 #pragma unroll
-    for (int q = 0; q < RT; ++q) {
-      lm_wait_vm<0>();
-      take_x(q);
-      asm volatile("" : "+v"(xr[q][0]), "+v"(xr[q][1]), "+v"(xr[q][2]), "+v"(xr[q][3]), "+v"(xr[q][4]),
-                   "+v"(xr[q][5]), "+v"(xr[q][6]), "+v"(xr[q][7]));  // read before the stage is loaded again
-      if (q + 2 < RT) load_x(q + 2);
-    }
+  for (int q = 0; q < RT; ++q) load_x(q);
+  lm_wait_vm<0>();
+#pragma unroll
+  for (int q = 0; q < RT; ++q) {
+    take_x(q);
+    asm volatile("" : "+v"(xr[q][0]), "+v"(xr[q][1]), "+v"(xr[q][2]), "+v"(xr[q][3]), "+v"(xr[q][4]),
+                 "+v"(xr[q][5]), "+v"(xr[q][6]), "+v"(xr[q][7]));  // read before the stage is loaded again
   }
 
   const int ntiles = (vocab + kLmSplitTile - 1) / kLmSplitTile;
   const auto load_tile = [&](int t, int stage) {
-    if (!on || t >= ntiles) return;
+    if (t >= ntiles) return;
     const uint64_t base = (uint64_t)(w + (int64_t)t * kLmSplitTile * w_stride + wave * kLmKChunk);
     const int last = vocab - 1 - t * kLmSplitTile;  // rows past the vocabulary re-read the last one
 #pragma unroll
@@ -369,9 +494,7 @@ __global__ __launch_bounds__(kLmSplitThreads, 2) void lm_head_split_kernel(
       lm_load16(base, (uint32_t)(min(4 * i + lrow, last) * (int)w_stride + (lchunk ^ (4 * (i & 3))) * 8) * 2,
                 slice0 + stage * kLmStageBytes + 1024 * i);
   };
-  unsigned long long best[kRounds];
-#pragma unroll
-  for (int p = 0; p < kRounds; ++p) best[p] = 0;
+  unsigned long long best = 0;
   load_tile(rank, 0);
   load_tile(rank + nrank, 1);
   int stage = 0;
@@ -381,76 +504,64 @@ __global__ __launch_bounds__(kLmSplitThreads, 2) void lm_head_split_kernel(
     for (int q = 0; q < RT; ++q)
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[q][i] = 0.f;
-    if (on) {
-      if (t + nrank < ntiles)
-        lm_wait_vm<8>();
-      else
-        lm_wait_vm<0>();
+    if (t + nrank < ntiles)
+      lm_wait_vm<8>();
+    else
+      lm_wait_vm<0>();
 #pragma unroll
-      for (int s8 = 0; s8 < 8; ++s8) {
-        const bf16x8_t av = __builtin_bit_cast(bf16x8_t, read(stage, s8));
+    for (int s8 = 0; s8 < 8; ++s8) {
+      const bf16x8_t av = __builtin_bit_cast(bf16x8_t, read(stage, s8));
 #pragma unroll
-        for (int q = 0; q < RT; ++q)
-          acc[q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, __builtin_bit_cast(bf16x8_t, xr[q][s8]), acc[q], 0, 0, 0);
-      }
+      for (int q = 0; q < RT; ++q)
+        acc[q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, __builtin_bit_cast(bf16x8_t, xr[q][s8]), acc[q], 0, 0, 0);
     }
     // D layout: lane holds hidden row 32 q + r and vocabulary rows 8 (i >> 2) + 4 h + (i & 3).
-    // Wavefront v sums quad v & 3 of row block 2 p + (v >> 2) over the slices, in K order.
+    // Wavefront v sums quad v & 3 of row block v >> 2 over the slices, in K order.
 #pragma unroll
-    for (int p = 0; p < kRounds; ++p) {
-      if (on) {
+    for (int q = 0; q < RT; ++q)
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          if (2 * p + q >= RT) break;
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<__attribute__((address_space(3))) f32x4_t*>(own + stage * kLmStageBytes + (4 * q + i) * 1024 +
+                                                                     lane * 16) =
+            f32x4_t{acc[q][4 * i], acc[q][4 * i + 1], acc[q][4 * i + 2], acc[q][4 * i + 3]};
+    lm_barrier();
+    if ((wave >> 2) < RT) {
+      const lds_char* const part = smem + stage * kLmStageBytes + wave * 1024 + lane * 16;
+      f32x4_t sum = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            *reinterpret_cast<__attribute__((address_space(3))) f32x4_t*>(own + stage * kLmStageBytes + (4 * q + i) * 1024 + lane * 16) =
-                f32x4_t{acc[2 * p + q][4 * i], acc[2 * p + q][4 * i + 1], acc[2 * p + q][4 * i + 2],
-                        acc[2 * p + q][4 * i + 3]};
-        }
+      for (int u0 = 0; u0 < kLmSplitWaves; u0 += 4) {
+        f32x4_t v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          v[u] = *reinterpret_cast<const __attribute__((address_space(3))) f32x4_t*>(part + (u0 + u) * kLmSliceBytes);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) sum += v[u];
       }
-      lm_barrier();
-      if (2 * p + (wave >> 2) < RT) {
-        const lds_char* const part = smem + stage * kLmStageBytes + wave * 1024 + lane * 16;
-        f32x4_t sum = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      const int vrow = t * kLmSplitTile + 8 * (wave & 3) + 4 * h;
 #pragma unroll
-        for (int u0 = 0; u0 < kLmSplitWaves; u0 += 4) {
-          f32x4_t v[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u)
-            v[u] = *reinterpret_cast<const __attribute__((address_space(3))) f32x4_t*>(part + min(u0 + u, nw - 1) * kLmSliceBytes);
-#pragma unroll
-          for (int u = 0; u < 4; ++u)
-            if (u0 + u < nw) sum += v[u];
+      for (int e = 0; e < 4; ++e)
+        if (vrow + e < vocab) {
+          const unsigned long long key = logit_key(round_to_bf16(sum[e]), (uint32_t)(vrow + e));
+          best = key > best ? key : best;
         }
-        const int vrow = t * kLmSplitTile + 8 * (wave & 3) + 4 * h;
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (vrow + e < vocab) {
-            const unsigned long long key = logit_key(round_to_bf16(sum[e]), (uint32_t)(vrow + e));
-            best[p] = key > best[p] ? key : best[p];
-          }
-      }
-      lm_barrier();
     }
+    lm_barrier();
     load_tile(t + 2 * nrank, stage);
   }
   // the best of a hidden row over its quads (wavefronts) and lane halves
-#pragma unroll
-  for (int p = 0; p < kRounds; ++p) {
-    const unsigned long long other = __shfl_xor(best[p], 32, kWave);
-    const unsigned long long b = other > best[p] ? other : best[p];
-    const int m = m0 + 32 * (2 * p + (wave >> 2)) + r;
-    if (h == 0 && 2 * p + (wave >> 2) < RT && m < rows && b != 0) atomicMax(keys + m, b);
-  }
+  const unsigned long long other = __shfl_xor(best, 32, kWave);
+  const unsigned long long b = other > best ? other : best;
+  const int m = 32 * (wave >> 2) + r;
+  if (h == 0 && (wave >> 2) < RT && m < rows && b != 0) atomicMax(keys + m, b);
 }
 
-// The same with four K slices of 256 columns and two halves of the hidden rows: wavefront
-// k + 4 m multiplies slice k by row blocks 2 m and 2 m + 1, so half as many partial sums meet, in
-// one round instead of two; the two wavefronts of a slice share it (and load half of its rows
-// each). Measured against lm_head_split_kernel (us, whole call): 65 rows 80.8 -> 79.2, 97 rows
-// 89.0 -> 79.5, 128 rows 89.5 -> 79.7. It takes more than kLmSplit4Rows hidden rows (below, a
-// second half would hold no rows) of a hidden size that its slices divide.
+// The same with four K slices of 256 columns and two halves of 128 hidden rows: wavefront k + 4 m
+// multiplies slice k by row blocks 2 m and 2 m + 1, so half as many partial sums meet; the two
+// wavefronts of a slice share it (and load half of its rows each). It takes more than kLmSplit4Rows
+// hidden rows (below, a second half would hold no rows) of a hidden size that its slices divide; with
+// three slices a quarter of the wavefronts idles. Whole call over 151936 vocabulary rows, us,
+// lm_head_resident_kernel -> this one: 96 rows 92.5 -> 80.7, 128 rows 94.3 -> 81.1, 129 rows 131.5 ->
+// 116.9, 512 rows 290.0 -> 218.6.
 constexpr int kLmSplit4Rows = 64;
 
 __global__ __launch_bounds__(kLmSplitThreads, 2) void lm_head_split4_kernel(
@@ -466,7 +577,9 @@ __global__ __launch_bounds__(kLmSplitThreads, 2) void lm_head_split4_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int ks = wave & 3, half_m = wave >> 2;
   const int r = lane & 31, h = lane >> 5;
-  const int j = blockIdx.x >> 3;  // see lm_head_split_kernel
+  // the `groups` work-groups of one place in the vocabulary walk (row groups of 128) have linear
+  // ids l, l + 8, ... and so share an XCD's L2
+  const int j = blockIdx.x >> 3;
   const int rg = j % groups;
   const int rank = (j / groups) * 8 + (blockIdx.x & 7);
   const int nrank = gridDim.x / groups;
@@ -634,6 +747,22 @@ hipError_t launch_silu_and_mul(const void* x, int64_t x_stride, int32_t rows, in
   return hipGetLastError();
 }
 
+// Whether the split kernels are the faster ones. A persistent work-group pays its start (the hidden
+// rows into registers, two tiles on their way) once for the tiles it walks, and a K slice without
+// columns is a wavefront without work. lm_head_resident_kernel / split kernels, time ratio by tiles per work-group (2.3, 4.6, 9.3, 18.5):
+//   hidden 1024, 1-64 rows     0.84-1.15  0.77-0.90  0.99-1.13  1.05-1.14
+//   hidden 1024, 65-128 rows   0.80-0.83  1.03-1.05  1.06-1.08  1.14-1.16
+//   hidden 1024, more rows     1.03-1.05  0.97-1.42  1.02-1.58  1.10-1.46
+//   hidden 768, 129-192 rows   0.87       0.81       0.85       0.90-0.94
+//   hidden 768, more rows      0.88-0.93  1.08-1.32  1.06-1.30  1.01-1.21
+// hidden 768 with fewer rows 0.67-1.02, hidden 512 0.53-0.92 and 128 0.30-0.69 (896: 0.71-1.20, not a
+// multiple of 256).
+bool lm_split_pays(int32_t rows, int32_t vocab, int32_t k_dim, int32_t groups, int32_t cus) {
+  const int64_t tiles = (int64_t)((vocab + kLmSplitTile - 1) / kLmSplitTile) * groups;
+  if (k_dim == kLmSplitHidden) return tiles >= (int64_t)cus * (rows <= kLmSplit4Rows ? 8 : rows <= kLmSplitRows ? 4 : 2);
+  return k_dim == kLmSplitHidden * 3 / 4 && rows > 3 * kLmSplitRows / 2 && tiles >= 4 * (int64_t)cus;
+}
+
 hipError_t launch_lm_head_greedy(const void* x, int64_t x_stride, const int32_t* cu_rows,
                                  const void* w, int64_t w_stride, int32_t rows, int32_t vocab,
                                  int32_t k_dim, unsigned long long* keys, int32_t* ids,
@@ -644,30 +773,32 @@ hipError_t launch_lm_head_greedy(const void* x, int64_t x_stride, const int32_t*
   const unsigned vt = (unsigned)((vocab + kLmVocabTile - 1) / kLmVocabTile);
   auto* xp = static_cast<const uint16_t*>(x);
   auto* wp = static_cast<const uint16_t*>(w);
-  if (k_dim <= kLmSplitMaxK && w_stride < (1 << 25)) {  // a tile's offsets fit 32 bits
-    static int cus_cached = 0;
-    if (cus_cached == 0) {
-      int dev = 0, cus = 0;
-      if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-        cus = 256;
-      cus_cached = cus;
-    }
-    const int groups = (rows + kLmSplitRows - 1) / kLmSplitRows;
-    const int per = 8 * groups;                      // one XCD round of every row group
-    int grid = (cus_cached / per) * per;
-    if (grid == 0) grid = per;
-    const int rt = groups > 1 ? 4 : (rows + 31) / 32;
-#define PK_LM_SPLIT(RT) \
-  hipLaunchKernelGGL(lm_head_split_kernel<RT>, dim3(grid), dim3(kLmSplitThreads), 0, stream, xp, x_stride, cu_rows, wp, w_stride, rows, vocab, k_dim, groups, keys)
-    if (rows > kLmSplit4Rows && k_dim % 256 == 0) {
-      hipLaunchKernelGGL(lm_head_split4_kernel, dim3(grid), dim3(kLmSplitThreads), 0, stream, xp, x_stride, cu_rows, wp, w_stride, rows, vocab, k_dim, groups, keys);
-    } else switch (rt) {
-      case 1: PK_LM_SPLIT(1); break;
-      case 2: PK_LM_SPLIT(2); break;
-      case 3: PK_LM_SPLIT(3); break;
-      default: PK_LM_SPLIT(4); break;
-    }
-#undef PK_LM_SPLIT
+  static int cus_cached = 0;
+  if (cus_cached == 0) {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+      cus = 256;
+    cus_cached = cus;
+  }
+  // a persistent grid of whole XCD rounds of every row group
+  const auto grid_of = [](int groups) { return std::max(cus_cached / (8 * groups), 1) * 8 * groups; };
+  const int split_groups = (rows + kLmSplitRows - 1) / kLmSplitRows;
+  // (a split tile's offsets fit 32 bits)
+  if (w_stride < (1 << 25) && lm_split_pays(rows, vocab, k_dim, split_groups, cus_cached)) {
+    const dim3 grid(grid_of(split_groups));
+    if (rows > kLmSplit4Rows)
+      hipLaunchKernelGGL(lm_head_split4_kernel, grid, dim3(kLmSplitThreads), 0, stream, xp, x_stride, cu_rows, wp, w_stride, rows, vocab, k_dim, split_groups, keys);
+    else if (rows > 32)
+      hipLaunchKernelGGL(lm_head_split_kernel<2>, grid, dim3(kLmSplitThreads), 0, stream, xp, x_stride, cu_rows, wp, w_stride, rows, vocab, keys);
+    else
+      hipLaunchKernelGGL(lm_head_split_kernel<1>, grid, dim3(kLmSplitThreads), 0, stream, xp, x_stride, cu_rows, wp, w_stride, rows, vocab, keys);
+  } else if (k_dim <= kLmResidentMaxK) {
+    const int groups = (rows + kLmResidentRows - 1) / kLmResidentRows;
+    const dim3 grid(grid_of(groups));
+    if (rows <= 32)
+      hipLaunchKernelGGL(lm_head_resident_kernel<1>, grid, dim3(kLmResidentThreads), 0, stream, xp, x_stride, cu_rows, wp, w_stride, rows, vocab, k_dim, groups, keys);
+    else
+      hipLaunchKernelGGL(lm_head_resident_kernel<2>, grid, dim3(kLmResidentThreads), 0, stream, xp, x_stride, cu_rows, wp, w_stride, rows, vocab, k_dim, groups, keys);
   } else if (rows <= 32) {
     hipLaunchKernelGGL(lm_head_greedy_kernel<1>, dim3(vt, 1), dim3(kLmThreads), 0, stream, xp, x_stride, cu_rows, wp, w_stride, rows, vocab, k_dim, keys);
   } else if (rows <= 64) {

@@ -120,3 +120,19 @@ def test_lm_head_greedy_row_blocks_and_k_slices(gpu, rows, vocab, hidden):
     hd = torch.empty(rows, hidden + 8, dtype=torch.bfloat16, device=gpu)[:, :hidden].copy_(h)
     got = pagedkv.lm_head_greedy(hd, wd)
     _greedy_check(got, h.contiguous(), w.contiguous())
+
+
+@pytest.mark.parametrize("hidden,rows,vocab", [
+    (1024, 1, 65536), (1024, 31, 65537), (1024, 32, 65567), (1024, 33, 70001), (1024, 64, 65536),   # eight K slices
+    (1024, 65, 32769), (1024, 97, 40000), (1024, 128, 32768), (1024, 129, 8193), (1024, 300, 10007),  # four
+    (768, 193, 16385), (768, 256, 20000), (768, 513, 8191),                                          # three of them
+    (1024, 64, 65504), (1024, 65, 32736), (1024, 129, 8160), (768, 192, 20000)])                     # below the lines
+def test_lm_head_greedy_split_kernels(gpu, hidden, rows, vocab):
+    """The calls that the split kernels take (vocabularies of several tiles per work-group, 256 of them), with
+    row blocks and vocabularies that end inside a tile, strided rows, and the first sizes on the other
+    side of each line."""
+    print(f"[lm-head] split rows={rows} vocab={vocab} hidden={hidden}", flush=True)
+    w, h = _rand((vocab, hidden), 31, 0.02), _rand((rows, hidden), 32 + rows)
+    wd = torch.empty(vocab, hidden + 64, dtype=torch.bfloat16, device=gpu)[:, :hidden].copy_(w)
+    hd = torch.empty(rows, hidden + 8, dtype=torch.bfloat16, device=gpu)[:, :hidden].copy_(h)
+    _greedy_check(pagedkv.lm_head_greedy(hd, wd), h, w)
