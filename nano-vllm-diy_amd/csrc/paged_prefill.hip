@@ -574,8 +574,8 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const AttnAr
 // prefill_kernel's, but an item starts sooner (no pipeline to fill, a third of the code to fetch
 // into a cold instruction cache), which decides where a work-group has one or two short items:
 // one item of 7 tiles per work-group 36.7 against 40.9 us a call, 15 chunks of 100 over 2048
-// keys 74.5 against 81.0. prefill_kernel is ahead from about 36 tiles per work-group (see
-// launch_prefill_gpc).
+// keys 74.5 against 81.0. prefill_kernel is ahead from about 34 tiles per work-group (see
+// small_prefill).
 constexpr int kW8Stages = 2;             // K and V LDS stages
 
 // One work item: kv head g of group `it` = (sequence b, query tile qt, key tiles [tb, te),
@@ -2154,19 +2154,31 @@ int device_prefill_slots() {
   return cached[dev];
 }
 
+// Which kernel a call takes, from its launch bounds (the lengths are on the device): an estimate of the
+// key tiles per work-group, with all `rows` query rows in sequences of the longest key count's half --
+// what the causal limit leaves of fresh rows, and half of the longest cached prefix for the others. The
+// w8 kernel starts an item sooner, prefill_kernel's tile takes less. Whole calls with `real` tiles per
+// work-group, time of w8 / time of prefill_kernel, with warm caches and with 512 MiB read before each
+// call (which evicts the kernels' code too):
+//   uniform paged chunks   real 5 0.92 / 0.90   9 0.93 / 0.92   18 0.96 / 0.95   33 1.00 / 0.97
+//                          36 1.02 / 1.02   41 1.03 / 1.02   63 1.01 / 1.02   73 1.05 / 1.03
+//                          129 1.09 / 1.08   274 1.11 / 1.11
+//   uniform fresh prompts  real 9 0.95 / 0.94   18 0.97 / 0.96   33 1.02 / 1.01   36 1.06 / 1.09   68 1.06 / 1.05
+//   ragged                 prompts of 100-1024 28 0.97 / 0.97, 34 1.00 / 0.99; of 100-512 21 0.95 / 0.94;
+//                          chunks of 512 over 0-4096 keys 24 0.96 / 0.96; of 128-1024 over 1024 38 1.06 / 1.06
+// so the line is near 34 real tiles; the estimate is up to a fifth above them for ragged fresh
+// prompts, and below them for chunks that all have the longest prefix (half at worst, which leaves
+// up to 3% where they lie between 36 and 72).
+constexpr int kSmallTiles = 36;
+template <int G>
+bool small_prefill(const AttnArgs& a, bool causal, int64_t rows) {
+  constexpr int TM = kPrefillRows / G;
+  const double keys = causal ? 0.5 * ((double)a.max_seqlen_k + TM) : (double)a.max_seqlen_k;
+  return (double)rows * a.num_kv_heads * keys < (double)kSmallTiles * a.pf_slots * TM * kTileKeys;
+}
+
 template <int G, bool PAGED, bool CAUSAL>
-hipError_t launch_prefill_gpc(const AttnArgs& a, hipStream_t stream) {
-  // Which kernel: the launch bounds' tiles per work-group, if every sequence were as long as they
-  // allow (the lengths are on the device). Uniform batches, w8 kernel against prefill_kernel (us
-  // per call). Paged: 15 tiles 60.8 / 63.0, 16 74.5 / 81.0, 20 81.4 / 81.5 and 79.6 / 81.5, 31
-  // 115.8 / 118.8, 36 114.9 / 111.7, 37 115.2 / 114.3, 48 124.0 / 119.9, 300 619 / 554. Flat (a
-  // prompt's tiles are half the bound): 4 39.7 / 41.1, 8 44.8 / 47.0, 16 103.6 / 104.8, 31 112.9 /
-  // 112.0, 32 77.4 / 79.4, 64 108.9 / 104.6, 256 315 / 288. A ragged batch is taken for a larger one: that costs
-  // at most the few us by which the small calls differ.
-  constexpr int kSmallTiles = 36;
-  const int64_t tiles = (int64_t)a.num_seqs * a.prefill_qtiles * ((a.max_seqlen_k + kTileKeys - 1) / kTileKeys) *
-                        a.num_kv_heads;
-  const bool small = tiles < (int64_t)kSmallTiles * a.pf_slots;
+hipError_t launch_prefill_gpc(const AttnArgs& a, bool small, hipStream_t stream) {
   if (small) {
     hipLaunchKernelGGL((prefill_plan_kernel<G, CAUSAL, true>), dim3(1), dim3(kPlanThreads), 0, stream, a);
     hipLaunchKernelGGL((prefill_w8_kernel<G, PAGED, CAUSAL>), dim3(a.pf_slots), dim3(kPrefillThreads), 0, stream, a);
@@ -2185,9 +2197,10 @@ hipError_t launch_prefill_g(const AttnArgs& a, bool paged, bool causal, int max_
   pa.prefill_qtiles = (max_seqlen_q + TM - 1) / TM;
   pa.pf_slots = device_prefill_slots();
   pa.flat_step = decode_flat_step(G, a.num_kv_heads);  // the decode pieces' step, for the merge kernel's combines
+  const bool small = small_prefill<G>(pa, causal, (int64_t)a.num_seqs * max_seqlen_q);
   if (paged)
-    return causal ? launch_prefill_gpc<G, true, true>(pa, stream) : launch_prefill_gpc<G, true, false>(pa, stream);
-  return causal ? launch_prefill_gpc<G, false, true>(pa, stream) : launch_prefill_gpc<G, false, false>(pa, stream);
+    return causal ? launch_prefill_gpc<G, true, true>(pa, small, stream) : launch_prefill_gpc<G, true, false>(pa, small, stream);
+  return causal ? launch_prefill_gpc<G, false, true>(pa, small, stream) : launch_prefill_gpc<G, false, false>(pa, small, stream);
 }
 
 }  // namespace

@@ -3,7 +3,7 @@ keys score hundreds above the first 32, far below them, or both, with overflow t
 softmax is then close to one-hot, and the fp32 oracle gives it), the merge of its splits, the range of V,
 rows past a sequence's end, and the edges of steps and tiles.
 
-Which kernel a call takes follows from its launch bounds (launch_prefill_gpc); a key-count bound of BOUND_K
+Which kernel a call takes follows from its launch bounds (small_prefill); a key-count bound of BOUND_K
 takes any call of this file to the pipelined one."""
 import pytest
 import torch
@@ -14,7 +14,7 @@ from paged_helpers import assert_close_bf16
 
 pytestmark = pytest.mark.gpu
 D = 128
-BOUND_K = 1 << 19
+BOUND_K = 1 << 21
 GROUPS = [(16, 8), (4, 4), (8, 2), (8, 1)]  # GQA groups 2, 1, 4, 8
 
 
@@ -52,8 +52,9 @@ def _run(gpu, q, k, v, seqs, paged, causal=True, bound=BOUND_K):
     allocation): a row read past a sequence's end makes its tile's outputs NaN."""
     hq, hkv, max_q = q.shape[1], k.shape[1], max(a for a, _ in seqs)
     max_k = bound or max(b for _, b in seqs)
-    if bound:  # 36 tiles per work-group of 256
-        assert len(seqs) * -(-max_q // (256 * hkv // hq)) * (max_k // 64) * hkv >= 36 * 256
+    if bound:  # an estimate of 36 tiles per work-group of 256, as small_prefill makes it
+        keys = (max_k + 256 * hkv // hq) / 2 if causal else max_k
+        assert sum(a for a, _ in seqs) * keys * hkv >= 36 * 256 * (256 * hkv // hq) * 64
     cu_q, cu_k = _cu([a for a, _ in seqs]).to(gpu), _cu([b for _, b in seqs]).to(gpu)
     if paged:
         kd, vd, bt = (x.to(gpu) for x in _paged(seqs, k, v, -(-max_k // 64)))
