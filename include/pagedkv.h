@@ -191,6 +191,28 @@ int pk_varlen_attention_shared_prefix(const void* q, int64_t q_row_stride,
                                       pk_stream_t stream);
 
 /*
+ * pk_varlen_attention_rows -- pk_varlen_attention_shared_prefix that is told how many query rows
+ * the call has. No counterpart in the reference. Same arguments, semantics and workspace; with
+ * the count a batch of decode rows and a few short chunks takes the kernel that is the faster
+ * one for it, where the other entry points have to assume max_seqlen_q rows of every sequence.
+ *   num_rows: the rows of q, cu_seqlens_q[num_seqs] or more (graph padding); 0: not known.
+ */
+int pk_varlen_attention_rows(const void* q, int64_t q_row_stride,
+                             const void* k, const void* v,
+                             int64_t k_row_stride, int64_t v_row_stride,
+                             int64_t k_block_stride, int64_t v_block_stride,
+                             const int32_t* block_table, int32_t block_table_stride,
+                             int32_t block_size,
+                             const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+                             int32_t num_seqs, int32_t max_seqlen_q, int32_t max_seqlen_k,
+                             int32_t num_heads, int32_t num_kv_heads, int32_t head_dim,
+                             float softmax_scale, int32_t causal,
+                             void* out, int64_t out_row_stride,
+                             void* workspace, size_t workspace_bytes,
+                             int32_t cached_prefix_keys, int32_t shared_prefix_keys,
+                             int64_t num_rows, pk_stream_t stream);
+
+/*
  * pk_varlen_attention_noalloc -- pk_varlen_attention_ex for callers that cannot allocate
  * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc). No
  * counterpart in the reference. Same arguments, semantics and kernels as

@@ -147,7 +147,7 @@ int check_linear(const char* what, const void* x, int64_t x_row_stride, const vo
 
 extern "C" {
 
-int pk_abi_version(void) { return 9; }
+int pk_abi_version(void) { return 10; }
 
 const char* pk_last_error(void) { return g_last_error.c_str(); }
 
@@ -251,7 +251,7 @@ int attention_impl(const void* q, int64_t q_row_stride, const void* k, const voi
                    int32_t max_seqlen_q, int32_t max_seqlen_k, int32_t num_heads, int32_t num_kv_heads,
                    int32_t head_dim, float softmax_scale, int32_t causal, void* out, int64_t out_row_stride,
                    void* workspace, size_t workspace_bytes, int32_t cached_prefix_keys, const FusedProducer* fp,
-                   int32_t shared_prefix_keys, pk_stream_t stream) {
+                   int32_t shared_prefix_keys, int64_t num_rows, pk_stream_t stream) {
   if (head_dim != pk::kHeadDim)
     return fail(PK_ERR_UNSUPPORTED, "varlen_attention: head_dim=%d not built (only %d)", head_dim, pk::kHeadDim);
   if (num_seqs < 0 || max_seqlen_q < 0 || max_seqlen_k < 0)
@@ -424,7 +424,7 @@ int attention_impl(const void* q, int64_t q_row_stride, const void* k, const voi
   }
   if (rc != PK_OK) return rc;
   if (max_seqlen_q > 1)
-    rc = hip_status(pk::launch_prefill(a, group, paged, causal != 0, max_seqlen_q, s), "prefill launch");
+    rc = hip_status(pk::launch_prefill(a, group, paged, causal != 0, max_seqlen_q, num_rows, s), "prefill launch");
   return rc;
 }
 
@@ -443,7 +443,7 @@ int pk_varlen_attention_ex(const void* q, int64_t q_row_stride, const void* k, c
   return attention_impl(q, q_row_stride, k, v, k_row_stride, v_row_stride, k_block_stride, v_block_stride,
                         block_table, block_table_stride, block_size, cu_seqlens_q, cu_seqlens_k, num_seqs,
                         max_seqlen_q, max_seqlen_k, num_heads, num_kv_heads, head_dim, softmax_scale, causal, out,
-                        out_row_stride, workspace, workspace_bytes, cached_prefix_keys, nullptr, 0, stream);
+                        out_row_stride, workspace, workspace_bytes, cached_prefix_keys, nullptr, 0, 0, stream);
 }
 
 int pk_varlen_attention_shared_prefix(const void* q, int64_t q_row_stride, const void* k, const void* v,
@@ -455,16 +455,34 @@ int pk_varlen_attention_shared_prefix(const void* q, int64_t q_row_stride, const
                                       int32_t num_kv_heads, int32_t head_dim, float softmax_scale, int32_t causal,
                                       void* out, int64_t out_row_stride, void* workspace, size_t workspace_bytes,
                                       int32_t cached_prefix_keys, int32_t shared_prefix_keys, pk_stream_t stream) {
+  return pk_varlen_attention_rows(q, q_row_stride, k, v, k_row_stride, v_row_stride, k_block_stride, v_block_stride,
+                                  block_table, block_table_stride, block_size, cu_seqlens_q, cu_seqlens_k, num_seqs,
+                                  max_seqlen_q, max_seqlen_k, num_heads, num_kv_heads, head_dim, softmax_scale,
+                                  causal, out, out_row_stride, workspace, workspace_bytes, cached_prefix_keys,
+                                  shared_prefix_keys, 0, stream);
+}
+
+int pk_varlen_attention_rows(const void* q, int64_t q_row_stride, const void* k, const void* v,
+                             int64_t k_row_stride, int64_t v_row_stride, int64_t k_block_stride,
+                             int64_t v_block_stride, const int32_t* block_table,
+                             int32_t block_table_stride, int32_t block_size,
+                             const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int32_t num_seqs,
+                             int32_t max_seqlen_q, int32_t max_seqlen_k, int32_t num_heads,
+                             int32_t num_kv_heads, int32_t head_dim, float softmax_scale, int32_t causal,
+                             void* out, int64_t out_row_stride, void* workspace, size_t workspace_bytes,
+                             int32_t cached_prefix_keys, int32_t shared_prefix_keys,
+                             int64_t num_rows, pk_stream_t stream) {
   g_last_error.clear();
   if (shared_prefix_keys < 0)
-    return fail(PK_ERR_INVALID_ARG, "varlen_attention_shared_prefix: shared_prefix_keys=%d < 0", shared_prefix_keys);
+    return fail(PK_ERR_INVALID_ARG, "varlen_attention: shared_prefix_keys=%d < 0", shared_prefix_keys);
   if (block_table == nullptr && shared_prefix_keys > 0)
-    return fail(PK_ERR_INVALID_ARG, "varlen_attention_shared_prefix: a shared prefix needs paged K/V (block_table)");
+    return fail(PK_ERR_INVALID_ARG, "varlen_attention: a shared prefix needs paged K/V (block_table)");
+  if (num_rows < 0) return fail(PK_ERR_INVALID_ARG, "varlen_attention: num_rows=%lld < 0", (long long)num_rows);
   return attention_impl(q, q_row_stride, k, v, k_row_stride, v_row_stride, k_block_stride, v_block_stride,
                         block_table, block_table_stride, block_size, cu_seqlens_q, cu_seqlens_k, num_seqs,
                         max_seqlen_q, max_seqlen_k, num_heads, num_kv_heads, head_dim, softmax_scale, causal, out,
                         out_row_stride, workspace, workspace_bytes, cached_prefix_keys, nullptr, shared_prefix_keys,
-                        stream);
+                        num_rows, stream);
 }
 
 int pk_qkv_decode_attention(const void* qkv, int64_t qkv_row_stride, const int64_t* positions,
@@ -497,7 +515,7 @@ int pk_qkv_decode_attention(const void* qkv, int64_t qkv_row_stride, const int64
   return attention_impl(nullptr, 0, k_cache, v_cache, k_row_stride, v_row_stride, k_block_stride, v_block_stride,
                         block_table, block_table_stride, block_size, cu_seqlens_q, cu_seqlens_k, num_seqs, 1,
                         max_seqlen_k, num_heads, num_kv_heads, head_dim, softmax_scale, 1, out, out_row_stride,
-                        workspace, workspace_bytes, cached_prefix_keys, &fp, 0, stream);
+                        workspace, workspace_bytes, cached_prefix_keys, &fp, 0, 0, stream);
 }
 
 int pk_store_decode_attention(const void* q, int64_t q_row_stride, const void* key, int64_t key_row_stride,
@@ -526,7 +544,7 @@ int pk_store_decode_attention(const void* q, int64_t q_row_stride, const void* k
   return attention_impl(q, q_row_stride, k_cache, v_cache, k_row_stride, v_row_stride, k_block_stride,
                         v_block_stride, block_table, block_table_stride, block_size, cu_seqlens_q, cu_seqlens_k,
                         num_seqs, 1, max_seqlen_k, num_heads, num_kv_heads, head_dim, softmax_scale, 1, out,
-                        out_row_stride, workspace, workspace_bytes, cached_prefix_keys, &fp, 0, stream);
+                        out_row_stride, workspace, workspace_bytes, cached_prefix_keys, &fp, 0, 0, stream);
 }
 
 int pk_qk_norm_rope_store(const void* qkv, int64_t qkv_row_stride, const int64_t* positions,
@@ -755,5 +773,5 @@ extern "C" int pk_varlen_attention_noalloc(const void* q, int64_t q_row_stride, 
   return attention_impl(q, q_row_stride, k, v, k_row_stride, v_row_stride, k_block_stride, v_block_stride, block_table,
                         block_table_stride, block_size, cu_seqlens_q, cu_seqlens_k, num_seqs, max_seqlen_q,
                         max_seqlen_k, num_heads, num_kv_heads, head_dim, softmax_scale, causal, out, out_row_stride,
-                        ws, need > 0 ? (size_t)PK_NOALLOC_SCRATCH_BYTES : 0, cached_prefix_keys, nullptr, 0, stream);
+                        ws, need > 0 ? (size_t)PK_NOALLOC_SCRATCH_BYTES : 0, cached_prefix_keys, nullptr, 0, 0, stream);
 }

@@ -218,8 +218,9 @@ bool launch_shared_prefix_flat(AttnArgs& a, int group, hipStream_t stream, hipEr
 // The decode launch's combine pass alone (after launch_shared_prefix_flat).
 hipError_t launch_decode_combine(const AttnArgs& a, int group, hipStream_t stream);
 // bf16-MFMA attention over sequences with more than one query row.
+// num_rows: query rows of the call (0: not known), for the choice of the kernel.
 hipError_t launch_prefill(const AttnArgs& a, int group, bool paged, bool causal,
-                          int max_seqlen_q, hipStream_t stream);
+                          int max_seqlen_q, int64_t num_rows, hipStream_t stream);
 // Split size (keys per work-group) the decode kernel uses for these launch bounds.
 int decode_split_tokens(int num_seqs, int max_seqlen_k);
 // Flat decode grid for these launch bounds: groups == 0 when the split grid is used.

@@ -2155,7 +2155,7 @@ int device_prefill_slots() {
 }
 
 // Which kernel a call takes, from its launch bounds (the lengths are on the device): an estimate of the
-// key tiles per work-group, with all `rows` query rows in sequences of the longest key count's half --
+// key tiles per work-group, with all `rows` prefill rows in sequences of the longest key count's half --
 // what the causal limit leaves of fresh rows, and half of the longest cached prefix for the others. The
 // w8 kernel starts an item sooner, prefill_kernel's tile takes less. Whole calls with `real` tiles per
 // work-group, time of w8 / time of prefill_kernel, with warm caches and with 512 MiB read before each
@@ -2170,6 +2170,17 @@ int device_prefill_slots() {
 // prompts, and below them for chunks that all have the longest prefix (half at worst, which leaves
 // up to 3% where they lie between 36 and 72).
 constexpr int kSmallTiles = 36;
+//
+// Prefill rows: the call's rows less one per sequence, plus one for each that can be a prefill sequence
+// of the longest length. (With every sequence at that length 128 decode rows beside 8 chunks of 100 over
+// 2048 keys took prefill_kernel: 182.1 / 192.4 us warm / cold, w8 175.9 / 180.3; beside one chunk of 64
+// over 4096 159.2 / 166.2, w8 156.3 / 161.3.)
+int64_t prefill_rows_of(int num_seqs, int max_seqlen_q, int64_t num_rows) {
+  if (num_rows <= 0) return (int64_t)num_seqs * max_seqlen_q;
+  const int64_t more = std::max<int64_t>(num_rows - num_seqs, 0);
+  return more + std::min<int64_t>(num_seqs, (more + max_seqlen_q - 2) / (max_seqlen_q - 1));
+}
+
 template <int G>
 bool small_prefill(const AttnArgs& a, bool causal, int64_t rows) {
   constexpr int TM = kPrefillRows / G;
@@ -2191,13 +2202,14 @@ hipError_t launch_prefill_gpc(const AttnArgs& a, bool small, hipStream_t stream)
 }
 
 template <int G>
-hipError_t launch_prefill_g(const AttnArgs& a, bool paged, bool causal, int max_seqlen_q, hipStream_t stream) {
+hipError_t launch_prefill_g(const AttnArgs& a, bool paged, bool causal, int max_seqlen_q, int64_t num_rows,
+                            hipStream_t stream) {
   constexpr int TM = kPrefillRows / G;
   AttnArgs pa = a;
   pa.prefill_qtiles = (max_seqlen_q + TM - 1) / TM;
   pa.pf_slots = device_prefill_slots();
   pa.flat_step = decode_flat_step(G, a.num_kv_heads);  // the decode pieces' step, for the merge kernel's combines
-  const bool small = small_prefill<G>(pa, causal, (int64_t)a.num_seqs * max_seqlen_q);
+  const bool small = small_prefill<G>(pa, causal, prefill_rows_of(a.num_seqs, max_seqlen_q, num_rows));
   if (paged)
     return causal ? launch_prefill_gpc<G, true, true>(pa, small, stream) : launch_prefill_gpc<G, true, false>(pa, small, stream);
   return causal ? launch_prefill_gpc<G, false, true>(pa, small, stream) : launch_prefill_gpc<G, false, false>(pa, small, stream);
@@ -2301,14 +2313,14 @@ hipError_t launch_shared_prefix(const AttnArgs& a, int group, hipStream_t stream
 }
 
 hipError_t launch_prefill(const AttnArgs& a, int group, bool paged, bool causal, int max_seqlen_q,
-                          hipStream_t stream) {
+                          int64_t num_rows, hipStream_t stream) {
   if (a.num_seqs <= 0 || max_seqlen_q <= 1) return hipSuccess;
   if (!a.pf_queue || !a.pf_items || !a.pf_merges || !a.pf_part_o || !a.pf_part_ml) return hipErrorInvalidValue;
   switch (group) {
-    case 1: return launch_prefill_g<1>(a, paged, causal, max_seqlen_q, stream);
-    case 2: return launch_prefill_g<2>(a, paged, causal, max_seqlen_q, stream);
-    case 4: return launch_prefill_g<4>(a, paged, causal, max_seqlen_q, stream);
-    case 8: return launch_prefill_g<8>(a, paged, causal, max_seqlen_q, stream);
+    case 1: return launch_prefill_g<1>(a, paged, causal, max_seqlen_q, num_rows, stream);
+    case 2: return launch_prefill_g<2>(a, paged, causal, max_seqlen_q, num_rows, stream);
+    case 4: return launch_prefill_g<4>(a, paged, causal, max_seqlen_q, num_rows, stream);
+    case 8: return launch_prefill_g<8>(a, paged, causal, max_seqlen_q, num_rows, stream);
     default: return hipErrorInvalidValue;
   }
 }

@@ -151,7 +151,7 @@ def varlen_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     C-ABI takes it); None takes one per call (or the reserved one under graph capture).
     shared_prefix_keys (an addition, paged mode): decode keys below it are computed once per
     shared cache block, the query rows of every sequence that holds the block in one MFMA
-    tile (pk_varlen_attention_shared_prefix); results stay within the attention tolerance.
+    tile (pk_varlen_attention_rows); results stay within the attention tolerance.
     None or 0: off.
     """
     nq, num_heads, head_dim = q.shape
@@ -211,14 +211,9 @@ def varlen_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
             scale, 1 if causal else 0,
             out.data_ptr(), out.stride(0),
             ws.data_ptr() if ws is not None else 0, ws.numel() if ws is not None else 0)
-    if shared_prefix_keys and block_table is not None:
-        hint = PK_CACHED_PREFIX_KEYS_DEFAULT if cached_prefix_keys is None else int(cached_prefix_keys)
-        check(lib().pk_varlen_attention_shared_prefix(*args, hint, int(shared_prefix_keys), _stream(q)),
-              "pk_varlen_attention_shared_prefix")
-    elif cached_prefix_keys is None:
-        check(lib().pk_varlen_attention(*args, _stream(q)), "pk_varlen_attention")
-    else:
-        check(lib().pk_varlen_attention_ex(*args, int(cached_prefix_keys), _stream(q)), "pk_varlen_attention_ex")
+    hint = PK_CACHED_PREFIX_KEYS_DEFAULT if cached_prefix_keys is None else int(cached_prefix_keys)
+    shared = int(shared_prefix_keys) if shared_prefix_keys and block_table is not None else 0
+    check(lib().pk_varlen_attention_rows(*args, hint, shared, nq, _stream(q)), "pk_varlen_attention_rows")
     return out
 
 

@@ -405,6 +405,26 @@ def test_no_alloc_refuses_bounds_beyond_its_scratch():
                                            0, 1, 1, HQ, HKV, HEAD_DIM, 0.088, 1, None, HQ * HEAD_DIM, 0, None) == 0
 
 
+def test_rows_entry_point_argument_checks():
+    """pk_varlen_attention_rows refuses a negative row count and what the shared-prefix call refuses,
+    before any launch; 0 sequences is a no-op."""
+    lib = _lib.lib()
+    fake = ctypes.c_void_p(0x10000)
+    row = HKV * HEAD_DIM
+    base = [fake, HQ * HEAD_DIM, fake, fake, row, row, BLOCK_SIZE * row, BLOCK_SIZE * row, fake, 32, BLOCK_SIZE,
+            fake, fake, 4, 64, 4096, HQ, HKV, HEAD_DIM, 0.088, 1, fake, HQ * HEAD_DIM, None, 0, 2048]
+    assert lib.pk_varlen_attention_rows(*base, 0, -1, None) == _lib.PK_ERR_INVALID_ARG
+    assert b"num_rows" in lib.pk_last_error()
+    assert lib.pk_varlen_attention_rows(*base, -1, 70, None) == _lib.PK_ERR_INVALID_ARG
+    flat = list(base)
+    flat[8] = None
+    assert lib.pk_varlen_attention_rows(*flat, 512, 70, None) == _lib.PK_ERR_INVALID_ARG
+    assert lib.pk_varlen_attention_rows(*base, 0, 70, None) == _lib.PK_ERR_WORKSPACE
+    empty = list(base)
+    empty[13] = 0
+    assert lib.pk_varlen_attention_rows(*empty, 0, 70, None) == _lib.PK_OK
+
+
 def test_shared_prefix_argument_checks():
     """pk_varlen_attention_shared_prefix refuses a negative bound and a shared prefix in flat
     mode (no block tables to share blocks through) before any launch; 0 sequences is a no-op."""
