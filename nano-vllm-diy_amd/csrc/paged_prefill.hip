@@ -992,7 +992,7 @@ __device__ __forceinline__ bf16x8 read_v(const lds_char* sV, const TileLanes& tl
 // wait states of an MFMA that it does not know, so the order of the stream provides them: a score
 // is read 16 MFMAs after the last that wrote it, P is used 16 MFMAs after its conversion, K, Q
 // and V operands come from LDS reads (which are waited for); pf_iteration's scheduling barriers
-// keep that order.
+// keep that order, and tests/test_prefill_stream.py checks it in the built code.
 // S += K Q^T with S in architectural registers, Q in architectural (row block 0) or accumulation
 // registers (row block 1).
 __device__ __forceinline__ void mfma_s(f32x16& s, const bf16x8& k, const bf16x8& q, bool first, int rb) {
