@@ -86,7 +86,7 @@ struct AttnArgs {
   int32_t sp_quads;
   // chunked-prefill work plan (workspace): a work item is (sequence, kv head, query tile,
   // key-tile range); items of one query tile that was split over several key ranges write
-  // fp32 partials that a merge pass combines.
+  // bf16 partials that a merge pass combines.
   int32_t* pf_queue;            // kPrefillQueueInts header: 8 claim counters, item / merge counts, split size
   int4* pf_items;               // [pf_item_cap] groups (b, qt, tile_begin | tile_end << 16, partial group);
                                 // item i = kv head i % Hkv of group i / Hkv

@@ -8,16 +8,16 @@
 // from fresh rows at cu_seqlens_k (flat, all-fresh prompts).
 //
 // Work unit: 256 query rows = TM = 256 / G query tokens x the G query heads of one kv
-// head g, so each K/V tile staged in LDS serves the whole GQA group. A work-group of four
-// wavefronts (one per SIMD, one work-group per CU, the whole register file) owns the unit; a
-// wavefront owns two blocks of 32 rows, each 32 consecutive tokens of one head (TM >= 32 for
-// every GQA group built).
+// head g, so each K/V tile staged in LDS serves the whole GQA group. Two kernels own units, one
+// work-group per CU: prefill_kernel with four wavefronts (one per SIMD, the whole register file) of
+// two blocks of 32 rows, and prefill_w8_kernel, for small calls, with eight of one block; a block is
+// 32 consecutive tokens of one head (TM >= 32 for every GQA group built).
 //
 // Three launches, all sized on the host without reading device memory:
 //   1. plan (one work-group): reads cu_seqlens_q/k, counts each unit's key tiles under
 //      its causal limit, picks a split size T = max(8, kSplitNum / kSplitDen x total tiles
 //      / pool) tiles and writes the work list: every unit longer than T is cut into equal
-//      key ranges. Long items come first (four length buckets, longest first).
+//      key ranges. Long items come first (eight length buckets, four for small calls).
 //   2. prefill (a persistent pool of one work-group per CU): each work-group starts on the item
 //      of its own index, then claims items from the sub-queue of its XCD (item i belongs to
 //      sub-queue i mod 8, which for 8 kv heads is kv head i mod 8, so a head's K/V stays in one
@@ -28,7 +28,7 @@
 // The split bounds the longest chain of dependent tiles (a long cached prefix would
 // otherwise keep one work-group busy long after the rest of the GPU has finished).
 //
-// Per step of 32 keys (half a tile), per wavefront and 32-row block:
+// prefill_kernel, per step of 32 keys (half a tile), per wavefront and 32-row block:
 //   S^T (32 keys x 32 rows) = K (32 x 128) . Q^T (128 x 32)    8 v_mfma_f32_32x32x16_bf16
 //   P = 2^(S - reference of the row) (a lane owns one query row)
 //   O^T (128 x 32)         += V^T (128 x 32) . P^T (32 x 32)   8 v_mfma_f32_32x32x16_bf16
@@ -568,6 +568,47 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const AttnAr
   }
 }
 
+// ---- Claims and item inputs, of both prefill kernels -----------------------------------------
+// Wavefront 0: the claimed index, or -1 once every sub-queue is exhausted (own: the work-group's own
+// sub-queue xcd may have items left; pend: what lane 0's claim on it returned). Stealing reads the
+// other seven counters at once (lanes 0..6) and takes from the first sub-queue after this one
+// that has items left; a claim that lost the race reads again. Counters only grow, so a stale
+// read never shows a sub-queue exhausted too early.
+__device__ __forceinline__ int claim_finish(const AttnArgs& a, int xcd, int num_items, int lane, bool& own, int pend) {
+  if (own) {
+    const int64_t cand = (int64_t)__builtin_amdgcn_readfirstlane(pend) * 8 + xcd;
+    if (cand < num_items) return (int)cand;
+    own = false;
+  }
+  for (;;) {
+    const int q = (xcd + 1 + lane) & 7;
+    const int c = lane < 7 ? __hip_atomic_load(&a.pf_queue[q * kPrefillQueueStride], __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT)
+                           : 0;
+    const uint64_t left = __builtin_amdgcn_ballot_w64(lane < 7 && (int64_t)c * 8 + q < num_items);
+    if (left == 0) return -1;
+    const int qs = (xcd + 1 + __builtin_ctzll(left)) & 7;
+    int r = 0;
+    if (lane == 0) r = atomicAdd(&a.pf_queue[qs * kPrefillQueueStride], 1);
+    const int64_t cand = (int64_t)__builtin_amdgcn_readfirstlane(r) * 8 + qs;
+    if (cand < num_items) return (int)cand;
+  }
+}
+// Item i's work-list group (lanes 0..3), sequence b's bounds (lanes 0..3: cu_q[b], cu_q[b + 1], cu_k[b],
+// cu_k[b + 1]) and its first 64 block-table entries (one per lane: a tile's block id is a readlane).
+__device__ __forceinline__ int load_group(const AttnArgs& a, int i, int lane) {
+  return lane < 4 ? reinterpret_cast<const int*>(a.pf_items)[(int64_t)(i / a.num_kv_heads) * 4 + lane] : 0;
+}
+__device__ __forceinline__ int load_bounds(const AttnArgs& a, int b, int lane) {
+  const int32_t* p = lane < 2 ? a.cu_q + b + lane : a.cu_k + b + (lane - 2);
+  return lane < 4 ? *p : 0;
+}
+template <bool PAGED>
+__device__ __forceinline__ int load_bt(const AttnArgs& a, int b, int lane) {
+  if constexpr (!PAGED) return 0;
+  return lane < min(a.bt_stride, kWave) ? a.block_table[(int64_t)b * a.bt_stride + lane] : 0;
+}
+
 // ---- Small calls ---------------------------------------------------------------------------
 // Eight wavefronts of one row block each (two per SIMD) in phases QK - softmax - PV per 64-key
 // tile, K and V through registers into two LDS stages. Its tile takes half as long again as
@@ -665,37 +706,38 @@ __device__ __forceinline__ void prefill_item_w8(const AttnArgs& a, const int4 it
   // compiler's wait counting assumed the Q loads could still be in flight in every iteration
   // and made each k-block's QK MFMA wait for the global loads issued before it -- tile n + 2's
   // staging loads -- exposing their latency in every tile.)
-  if (ntiles <= 0) lds_barrier();
-  else {
-  load_tile_regs<PAGED>(a, b, k0, Lk, g, bt_lane, wave, lane, tbase, ll, R);
-  store_tile_lds(R, KS[0], VS[0], wave, lane);
-  if (ntiles > 1) load_tile_regs<PAGED>(a, b, k0, Lk, g, bt_lane, wave, lane, tbase + TN, ll, R);
-  lds_barrier();
-  for (int n0 = 0; n0 < ntiles; n0 += 2) {
+  if (ntiles <= 0) {
+    lds_barrier();
+  } else {
+    load_tile_regs<PAGED>(a, b, k0, Lk, g, bt_lane, wave, lane, tbase, ll, R);
+    store_tile_lds(R, KS[0], VS[0], wave, lane);
+    if (ntiles > 1) load_tile_regs<PAGED>(a, b, k0, Lk, g, bt_lane, wave, lane, tbase + TN, ll, R);
+    lds_barrier();
+    for (int n0 = 0; n0 < ntiles; n0 += 2) {
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int n = n0 + s;
-      if (n >= ntiles) break;
-      if (n == ntiles - 1) last_step();
-      const int t0 = tbase + n * TN;
-      // tile n + 1 (loaded during tile n - 1) goes to the other stage -- last read at step
-      // n - 1, before the previous barrier -- and its registers take tile n + 2's loads: one
-      // set of staging registers (a second set, holding tile n + 2 while tile n + 1 waited to
-      // be stored after tile n, took the kernel to 256 VGPRs with spills; 2.4% slower)
-      if (n + 1 < ntiles) {
-        store_tile_lds(R, KS[s ^ 1], VS[s ^ 1], wave, lane);
-        if (n + 2 < ntiles) load_tile_regs<PAGED>(a, b, k0, Lk, g, bt_lane, wave, lane, t0 + 2 * TN, ll, R);
-      }
-      bool any = false, full[kRowBlocks];
+      for (int s = 0; s < 2; ++s) {
+        const int n = n0 + s;
+        if (n >= ntiles) break;
+        if (n == ntiles - 1) last_step();
+        const int t0 = tbase + n * TN;
+        // tile n + 1 (loaded during tile n - 1) goes to the other stage -- last read at step
+        // n - 1, before the previous barrier -- and its registers take tile n + 2's loads: one
+        // set of staging registers (a second set, holding tile n + 2 while tile n + 1 waited to
+        // be stored after tile n, took the kernel to 256 VGPRs with spills; 2.4% slower)
+        if (n + 1 < ntiles) {
+          store_tile_lds(R, KS[s ^ 1], VS[s ^ 1], wave, lane);
+          if (n + 2 < ntiles) load_tile_regs<PAGED>(a, b, k0, Lk, g, bt_lane, wave, lane, t0 + 2 * TN, ll, R);
+        }
+        bool any = false, full[kRowBlocks];
 #pragma unroll
-      for (int rb = 0; rb < kRowBlocks; ++rb) {
-        any |= t0 <= lim_hi[rb];
-        full[rb] = t0 + TN - 1 <= lim_lo[rb];
+        for (int rb = 0; rb < kRowBlocks; ++rb) {
+          any |= t0 <= lim_hi[rb];
+          full[rb] = t0 + TN - 1 <= lim_lo[rb];
+        }
+        if (any) compute_tile(KS[s], VS[s], tl, qb, o, m_i, l_i, t0, lim, full, a.scale_log2, lane);
+        lds_barrier();
       }
-      if (any) compute_tile(KS[s], VS[s], tl, qb, o, m_i, l_i, t0, lim, full, a.scale_log2, lane);
-      lds_barrier();
     }
-  }
   }
 
   after_tiles();
@@ -771,60 +813,25 @@ __global__ __launch_bounds__(kPrefillThreads, kWavesPerSimd) void prefill_w8_ker
   const auto claim_issue = [&]() {
     if (wave == 0 && own && lane == 0) pend = atomicAdd(&a.pf_queue[xcd * kPrefillQueueStride], 1);
   };
-  // Wavefront 0: the claimed index, or -1 once every sub-queue is exhausted. Stealing reads
-  // the other seven counters at once (lanes 0..6) and takes from the first sub-queue after
-  // this one that has items left; a claim that lost the race reads again. Counters only
-  // grow, so a stale read never shows a sub-queue exhausted too early.
-  const auto claim_finish = [&]() {
-    if (own) {
-      const int64_t cand = (int64_t)__builtin_amdgcn_readfirstlane(pend) * 8 + xcd;
-      if (cand < num_items) return (int)cand;
-      own = false;
-    }
-    for (;;) {
-      const int q = (xcd + 1 + lane) & 7;
-      const int c = lane < 7 ? __hip_atomic_load(&a.pf_queue[q * kPrefillQueueStride], __ATOMIC_RELAXED,
-                                                 __HIP_MEMORY_SCOPE_AGENT)
-                             : 0;
-      const uint64_t left = __builtin_amdgcn_ballot_w64(lane < 7 && (int64_t)c * 8 + q < num_items);
-      if (left == 0) return -1;
-      const int qs = (xcd + 1 + __builtin_ctzll(left)) & 7;
-      int r = 0;
-      if (lane == 0) r = atomicAdd(&a.pf_queue[qs * kPrefillQueueStride], 1);
-      const int64_t cand = (int64_t)__builtin_amdgcn_readfirstlane(r) * 8 + qs;
-      if (cand < num_items) return (int)cand;
-    }
-  };
   // The next item's inputs load in two dependent steps around the current item's epilogue:
   // its work-list group (lanes 0..3) before the epilogue's stores, then the sequence's
   // bounds (lanes 0..3: cu_q[b], cu_q[b + 1], cu_k[b], cu_k[b + 1]) and first 64
   // block-table entries (one per lane: a tile's block id is a readlane, not a dependent
   // global load) after them.
-  const auto load_group = [&](int i) {
-    return lane < 4 ? reinterpret_cast<const int*>(a.pf_items)[(int64_t)(i / a.num_kv_heads) * 4 + lane] : 0;
-  };
   // The work list is trusted only as far as the buffers reach: a group naming a sequence
   // outside this call (a workspace overwritten by an overlapping call) reads sequence 0's
-  // bounds and is skipped by prefill_item.
+  // bounds and is skipped by prefill_item_w8.
   const auto seq_of = [&](int grpv) {
     const int b = __builtin_amdgcn_readlane(grpv, 0);
     return b >= 0 && b < a.num_seqs ? b : 0;
-  };
-  const auto load_bounds = [&](int b) {
-    const int32_t* p = lane < 2 ? a.cu_q + b + lane : a.cu_k + b + (lane - 2);
-    return lane < 4 ? *p : 0;
-  };
-  const auto load_bt = [&](int b) {
-    if constexpr (!PAGED) return 0;
-    return lane < min(a.bt_stride, kWave) ? a.block_table[(int64_t)b * a.bt_stride + lane] : 0;
   };
   // the first item is the work-group's own (item blockIdx), as in prefill_kernel
   int idx = (int)blockIdx.x < num_items ? (int)blockIdx.x : -1;
   int grpv = 0, cuv = 0, btv = 0;
   if (idx >= 0) {
-    grpv = load_group(idx);
-    cuv = load_bounds(seq_of(grpv));
-    btv = load_bt(seq_of(grpv));
+    grpv = load_group(a, idx, lane);
+    cuv = load_bounds(a, seq_of(grpv), lane);
+    btv = load_bt<PAGED>(a, seq_of(grpv), lane);
   }
   while (idx >= 0) {
     int next = -1, next_grpv = 0, next_cuv = 0, next_btv = 0;
@@ -842,17 +849,17 @@ __global__ __launch_bounds__(kPrefillThreads, kWavesPerSimd) void prefill_w8_ker
           // s_item was last read before this item's first barrier
           if (wave == 0) {
             if (!claimed) claim_issue();
-            const int c = claim_finish();
+            const int c = claim_finish(a, xcd, num_items, lane, own, pend);
             if (lane == 0) s_item = c;
           }
           lds_barrier();
           next = __builtin_amdgcn_readfirstlane(s_item);
-          if (next >= 0) next_grpv = load_group(next);
+          if (next >= 0) next_grpv = load_group(a, next, lane);
         },
         [&]() {
           if (next >= 0) {
-            next_cuv = load_bounds(seq_of(next_grpv));
-            next_btv = load_bt(seq_of(next_grpv));
+            next_cuv = load_bounds(a, seq_of(next_grpv), lane);
+            next_btv = load_bt<PAGED>(a, seq_of(next_grpv), lane);
           }
         });
     idx = next;
@@ -1330,41 +1337,6 @@ __global__ __launch_bounds__(kPfThreads, 1) void prefill_kernel(const AttnArgs a
       pend = atomicAdd(&a.pf_queue[xcd * kPrefillQueueStride + z], 1);
     }
   };
-  // Wavefront 0: the claimed index, or -1 once every sub-queue is exhausted. Stealing reads
-  // the other seven counters at once (lanes 0..6) and takes from the first sub-queue after
-  // this one that has items left; a claim that lost the race reads again. Counters only
-  // grow, so a stale read never shows a sub-queue exhausted too early.
-  const auto claim_finish = [&]() {
-    if (own) {
-      const int64_t cand = (int64_t)__builtin_amdgcn_readfirstlane(pend) * 8 + xcd;
-      if (cand < num_items) return (int)cand;
-      own = false;
-    }
-    for (;;) {
-      const int q = (xcd + 1 + lane) & 7;
-      const int c = lane < 7 ? __hip_atomic_load(&a.pf_queue[q * kPrefillQueueStride], __ATOMIC_RELAXED,
-                                                 __HIP_MEMORY_SCOPE_AGENT)
-                             : 0;
-      const uint64_t left = __builtin_amdgcn_ballot_w64(lane < 7 && (int64_t)c * 8 + q < num_items);
-      if (left == 0) return -1;
-      const int qs = (xcd + 1 + __builtin_ctzll(left)) & 7;
-      int r = 0;
-      if (lane == 0) r = atomicAdd(&a.pf_queue[qs * kPrefillQueueStride], 1);
-      const int64_t cand = (int64_t)__builtin_amdgcn_readfirstlane(r) * 8 + qs;
-      if (cand < num_items) return (int)cand;
-    }
-  };
-  const auto load_group = [&](int i) {
-    return lane < 4 ? reinterpret_cast<const int*>(a.pf_items)[(int64_t)(i / a.num_kv_heads) * 4 + lane] : 0;
-  };
-  const auto load_bounds = [&](int b) {
-    const int32_t* p = lane < 2 ? a.cu_q + b + lane : a.cu_k + b + (lane - 2);
-    return lane < 4 ? *p : 0;
-  };
-  const auto load_bt = [&](int b) {  // the first 64 block-table entries, one per lane
-    if constexpr (!PAGED) return 0;
-    return lane < min(a.bt_stride, kWave) ? a.block_table[(int64_t)b * a.bt_stride + lane] : 0;
-  };
   // The next item's inputs, in three steps over the current item's last tiles, each begun at the
   // top of a tile and ended at its bottom, so that none of the dependent round trips is waited
   // out: 0 the claim, published by wavefront 0; 1 the work-list entry; 2 the sequence's bounds
@@ -1376,11 +1348,11 @@ __global__ __launch_bounds__(kPfThreads, 1) void prefill_kernel(const AttnArgs a
       claim_issue();
     } else if (s == 1) {
       next = __builtin_amdgcn_readfirstlane(s_item);
-      if (next >= 0) gv = load_group(next);
+      if (next >= 0) gv = load_group(a, next, lane);
     } else if (s == 2 && next >= 0) {
       const int b = ng.x >= 0 && ng.x < a.num_seqs ? ng.x : 0;  // see make_item
-      cv = load_bounds(b);
-      btn = load_bt(b);
+      cv = load_bounds(a, b, lane);
+      btn = load_bt<PAGED>(a, b, lane);
     }
   };
   const auto lanes4 = [&](int v) {
@@ -1390,7 +1362,7 @@ __global__ __launch_bounds__(kPfThreads, 1) void prefill_kernel(const AttnArgs a
   const auto next_end = [&](int s) {
     if (s == 0) {
       if (wave == 0) {
-        const int c = claim_finish();
+        const int c = claim_finish(a, xcd, num_items, lane, own, pend);
         if (lane == 0) s_item = c;
       }
     } else if (s == 1) {
@@ -1410,7 +1382,7 @@ __global__ __launch_bounds__(kPfThreads, 1) void prefill_kernel(const AttnArgs a
   // The first item is the work-group's own (item blockIdx): no claim, and its work-list entry
   // loads with the item count (the list has room for more groups than there are work-groups).
   next = (int)blockIdx.x;
-  ng = lanes4(load_group(next));
+  ng = lanes4(load_group(a, next, lane));
   if (next >= num_items) return;
   next_begin(2);
   next_end(2);
@@ -1573,7 +1545,7 @@ __global__ __launch_bounds__(kPfThreads, 1) void prefill_kernel(const AttnArgs a
       // body 0: the scores of steps 0 and 1, the first softmax
       stage(0);
       if (nw > 0) {
-bf16x8 k[16];
+        bf16x8 k[16];
 #pragma unroll
         for (int j = 0; j < kPfAhead; ++j) k[j] = read_k(smem + k0s, tl, j);
 #pragma unroll
@@ -1639,11 +1611,12 @@ bf16x8 k[16];
       for (; n <= ntiles; ++n, t0 += TN) {
         stage(n);
         if (2 * n - 2 < nw) {
-        const lds_char* const ks = smem + k0s;
-        const lds_char* const vs = smem + v1s;
-        pf_iteration<1, true, false>(st, ks, ks + 32 * kRowBytes, vs, tl, t0, lim, a.scale_log2, half, nullptr, koff, 0);
-        pf_iteration<0, true, false>(st, ks + 32 * kRowBytes, smem + k1s, vs + 32 * kRowBytes, tl, t0 + kStepKeys, lim,
-                                     a.scale_log2, half, nullptr, koff, 0);
+          const lds_char* const ks = smem + k0s;
+          const lds_char* const vs = smem + v1s;
+          pf_iteration<1, true, false>(st, ks, ks + 32 * kRowBytes, vs, tl, t0, lim, a.scale_log2, half, nullptr, koff,
+                                       0);
+          pf_iteration<0, true, false>(st, ks + 32 * kRowBytes, smem + k1s, vs + 32 * kRowBytes, tl, t0 + kStepKeys,
+                                       lim, a.scale_log2, half, nullptr, koff, 0);
         }
         finish(n);
       }
