@@ -870,10 +870,10 @@ __global__ __launch_bounds__(kPrefillThreads, kWavesPerSimd) void prefill_w8_ker
 }
 
 // ---- The prefill kernel's tile loop --------------------------------------------------------
-// What bounded the loop before (eight wavefronts of one row block, phases QK - softmax - PV with
-// a barrier per tile, 4600 cycles per 64-key tile for 2048 cycles of MFMA): the two wavefronts of
-// a SIMD passed the phases together, so the MFMA, vector and LDS work added up, and every
-// wavefront read the whole tile from LDS (256 KiB per tile and CU at 128 B per cycle: as long as
+// What bounds the other kernel's loop (eight wavefronts of one row block, phases QK - softmax - PV
+// with a barrier per tile, for 2048 cycles of MFMA per 64-key tile): the two wavefronts of
+// a SIMD pass the phases together, so the MFMA, vector and LDS work add up, and every
+// wavefront reads the whole tile from LDS (256 KiB per tile and CU at 128 B per cycle: as long as
 // the MFMAs). Two row blocks per wavefront halve the LDS reads, and one wavefront per SIMD has
 // the registers (O 128, Q 64, two steps' scores 64 and P 32) to run three steps' parts beside
 // each other. What the loop then needs, measured per instruction (cycles, one wavefront): an MFMA
@@ -882,12 +882,11 @@ __global__ __launch_bounds__(kPrefillThreads, kWavesPerSimd) void prefill_w8_ker
 // v_dot2 (which the MFMA pipe executes too) 17, an LDS read beside a full slot 4. Hence: no
 // instruction uses a result of its own slot; sums by a small MFMA, not v_dot2; no running max (one
 // reference per row and item with 2^120 of room, checked by the sum at the end); K and V bypass
-// the registers. Steady tile 4600 -> 3000 cycles; 16 chunks of 1024 over 4096-token prefixes
-// (618 GFLOP) 647-670 -> 584-617 us per call with the 24 us store (kernel alone 692 -> 591 us in a
-// trace), at a clock that now falls with the load: an 8192^3 matrix product of the vendor's
-// library reaches 1.21 PFLOP/s here. A mixed step of 128 decodes and 8 chunks of 512 302.7 ->
-// 300.3 us, 31 dense prompts of 16384 tokens 150.9 -> 149.8 us: short items are bound by their
-// start and end (about 20000 of an average item's 45000 cycles).
+// the registers. 16 chunks of 1024 over 4096-token prefixes (618 GFLOP), item starts and ends
+// included: 4982 -> 4160 cycles per tile, MFMA pipes busy 43.6 -> 55.8% (counters), 650-671 -> 587-625 us
+// per call with the 24 us store, at a clock that falls with the load (1.93 GHz, less after several
+// such calls): an 8192^3 matrix product of the vendor's library reaches 1.21 PFLOP/s here. Short items
+// are bound by their start and end, so 31 dense prompts of 16384 tokens take 149.8 -> 148.8-151.3 us.
 constexpr int kPfWaves = 4;                      // one wavefront per SIMD, 64 query rows each
 constexpr int kPfThreads = kPfWaves * kWave;
 constexpr int kPfRB = kPrefillRows / (32 * kPfWaves);  // 32-row blocks per wavefront
