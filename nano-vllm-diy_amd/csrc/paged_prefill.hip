@@ -886,7 +886,7 @@ __global__ __launch_bounds__(kPrefillThreads, kWavesPerSimd) void prefill_w8_ker
 // included: 4982 -> 4160 cycles per tile, MFMA pipes busy 43.6 -> 55.8% (counters), 650-671 -> 587-625 us
 // per call with the 24 us store, at a clock that falls with the load (1.93 GHz, less after several
 // such calls): an 8192^3 matrix product of the vendor's library reaches 1.21 PFLOP/s here. Short items
-// are bound by their start and end, so 31 dense prompts of 16384 tokens take 149.8 -> 148.8-151.3 us.
+// are bound by their start and end, so calls of few tiles keep the other kernel (small_prefill).
 constexpr int kPfWaves = 4;                      // one wavefront per SIMD, 64 query rows each
 constexpr int kPfThreads = kPfWaves * kWave;
 constexpr int kPfRB = kPrefillRows / (32 * kPfWaves);  // 32-row blocks per wavefront
@@ -2141,9 +2141,11 @@ int device_prefill_slots() {
 //   uniform fresh prompts  real 9 0.95 / 0.94   18 0.97 / 0.96   33 1.02 / 1.01   36 1.06 / 1.09   68 1.06 / 1.05
 //   ragged                 prompts of 100-1024 28 0.97 / 0.97, 34 1.00 / 0.99; of 100-512 21 0.95 / 0.94;
 //                          chunks of 512 over 0-4096 keys 24 0.96 / 0.96; of 128-1024 over 1024 38 1.06 / 1.06
-// so the line is near 34 real tiles; the estimate is up to a fifth above them for ragged fresh
-// prompts, and below them for chunks that all have the longest prefix (half at worst, which leaves
-// up to 3% where they lie between 36 and 72).
+// so the line is near 34 real tiles. Fresh prompts of many lengths (flat K/V: their mean is known) count
+// with the middle of the mean and the longest, where the longest alone came out a fifth above their
+// tiles (31 prompts of 100-1024 took prefill_kernel: 151.7 us, w8 150.0, with the store); chunks that all
+// have the longest prefix come out below theirs (half at worst, which leaves up to 3% where they lie
+// between 36 and 72).
 constexpr int kSmallTiles = 36;
 //
 // Prefill rows: the call's rows less one per sequence, plus one for each that can be a prefill sequence
@@ -2157,9 +2159,12 @@ int64_t prefill_rows_of(int num_seqs, int max_seqlen_q, int64_t num_rows) {
 }
 
 template <int G>
-bool small_prefill(const AttnArgs& a, bool causal, int64_t rows) {
+bool small_prefill(const AttnArgs& a, bool paged, bool causal, int max_seqlen_q, int64_t num_rows) {
   constexpr int TM = kPrefillRows / G;
-  const double keys = causal ? 0.5 * ((double)a.max_seqlen_k + TM) : (double)a.max_seqlen_k;
+  const int64_t rows = prefill_rows_of(a.num_seqs, max_seqlen_q, num_rows);
+  double keys = a.max_seqlen_k;
+  if (!paged && num_rows > 0) keys = 0.5 * (keys + std::min(keys, (double)num_rows / a.num_seqs));
+  if (causal) keys = 0.5 * (keys + TM);
   return (double)rows * a.num_kv_heads * keys < (double)kSmallTiles * a.pf_slots * TM * kTileKeys;
 }
 
@@ -2184,7 +2189,7 @@ hipError_t launch_prefill_g(const AttnArgs& a, bool paged, bool causal, int max_
   pa.prefill_qtiles = (max_seqlen_q + TM - 1) / TM;
   pa.pf_slots = device_prefill_slots();
   pa.flat_step = decode_flat_step(G, a.num_kv_heads);  // the decode pieces' step, for the merge kernel's combines
-  const bool small = small_prefill<G>(pa, causal, prefill_rows_of(a.num_seqs, max_seqlen_q, num_rows));
+  const bool small = small_prefill<G>(pa, paged, causal, max_seqlen_q, num_rows);
   if (paged)
     return causal ? launch_prefill_gpc<G, true, true>(pa, small, stream) : launch_prefill_gpc<G, true, false>(pa, small, stream);
   return causal ? launch_prefill_gpc<G, false, true>(pa, small, stream) : launch_prefill_gpc<G, false, false>(pa, small, stream);

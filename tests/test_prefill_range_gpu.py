@@ -53,7 +53,8 @@ def _run(gpu, q, k, v, seqs, paged, causal=True, bound=BOUND_K):
     hq, hkv, max_q = q.shape[1], k.shape[1], max(a for a, _ in seqs)
     max_k = bound or max(b for _, b in seqs)
     if bound:  # an estimate of 36 tiles per work-group of 256, as small_prefill makes it
-        keys = (max_k + 256 * hkv // hq) / 2 if causal else max_k
+        keys = max_k if paged else (max_k + sum(a for a, _ in seqs) / len(seqs)) / 2
+        keys = (keys + 256 * hkv // hq) / 2 if causal else keys
         assert sum(a for a, _ in seqs) * keys * hkv >= 36 * 256 * (256 * hkv // hq) * 64
     cu_q, cu_k = _cu([a for a, _ in seqs]).to(gpu), _cu([b for _, b in seqs]).to(gpu)
     if paged:
